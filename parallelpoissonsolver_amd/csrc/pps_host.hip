@@ -120,6 +120,8 @@ struct Ctx {
     int cheb_pairs = 1;  // Chebyshev sweeps run two per pass (k_cheb_pair)
     int deferred_x = 1;  // Krylov stages keep a ring of directions where the device holds it
     int cheb_kz = 0;     // z-chunk of the fused Chebyshev pair (0: chosen per launch)
+    double* stage_d = nullptr;  // dense planes on their way between pageable host memory and a pitched field
+    int stage_planes = 0;
     std::string err;
     std::shared_ptr<NNPrecond> nn;  // learned preconditioner of PPS_NN stages (pps_nn_attach)
     int fallback_switches = 0;      // FCG stages that switched to the fallback, this solve
@@ -1339,6 +1341,96 @@ static int build_chain(Ctx& C, const pps_stage* chain, int n, std::vector<std::u
 
 static Ctx* as_ctx(void* p) { return static_cast<Ctx*>(p); }
 
+static int field_of(Ctx& C, int id, Field& f)
+{
+    if (id < 0 || id >= PPS_NUM_FIELDS) return C.fail(PPS_ERR_ARG, "bad field id %d", id);
+    if (!C.fields[id].p) {
+        int rc = C.alloc_field(C.fields[id], 64);
+        if (rc) return rc;
+    }
+    f = C.fields[id];
+    return PPS_OK;
+}
+
+// `nk` planes of a pitched field from (UP) or to a dense block of guarded
+// planes, one wavefront per row
+template <bool UP>
+__global__ __launch_bounds__(256) void k_repitch(double* __restrict__ dense, double* __restrict__ field, Layout L,
+                                                 int k0, long long rows)
+{
+    const int lane = threadIdx.x & 63;
+    for (long long w = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); w < rows; w += (long long)gridDim.x * 4) {
+        double* d = dense + w * L.ng[0];
+        double* f = field + L.at(0, (int)(w % L.ng[1]), k0 + (int)(w / L.ng[1]));
+        for (int i = lane; i < L.ng[0]; i += 64) {
+            if constexpr (UP) f[i] = d[i];
+            else d[i] = f[i];
+        }
+    }
+}
+
+// whether `host` is ordinary pageable memory (not allocated or registered through HIP)
+static bool pageable(const void* host)
+{
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, host) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return at.type == hipMemoryTypeUnregistered;
+}
+
+// host array <-> field.  Pinned memory takes one pitched copy (57 GB/s, the
+// link's rate).  The same copy on pageable memory goes row by row, about 9 us
+// each way per row (132^3: 158 ms up, 119 ms down); there, dense blocks of
+// planes are copied into a device buffer of at most kStageBytes (or one plane)
+// and a kernel moves them to the pitched rows: 0.6 ms up, 1.1 ms down.
+constexpr size_t kStageBytes = 64u << 20;
+static int transfer(Ctx& C, int field, double* host, bool up)
+{
+    Field f;
+    int rc = field_of(C, field, f);
+    if (rc) return rc;
+    const size_t plane = (size_t)C.ng[0] * C.ng[1];
+    const bool staged = pageable(host);
+    if (staged && !C.stage_d) {
+        const int np = (int)std::min<size_t>(C.ng[2], std::max<size_t>(1, kStageBytes / (plane * sizeof(double))));
+        if (hipMalloc(&C.stage_d, np * plane * sizeof(double)) == hipSuccess) {
+            C.stage_planes = np;
+        } else {
+            (void)hipGetLastError();  // no room: the row-by-row copy below still works
+            C.stage_d = nullptr;
+        }
+    }
+    if (staged && C.stage_d) {
+        for (int k0 = 0; k0 < C.ng[2]; k0 += C.stage_planes) {
+            const int nk = std::min(C.stage_planes, C.ng[2] - k0);
+            const size_t bytes = nk * plane * sizeof(double);
+            const long long rows = (long long)nk * C.ng[1];
+            const dim3 grid((unsigned)std::min<long long>((rows + 3) / 4, 8192));
+            double* h = host + k0 * plane;
+            if (up) {
+                if ((rc = C.hip(hipMemcpyAsync(C.stage_d, h, bytes, hipMemcpyHostToDevice, C.stream), "upload"))) return rc;
+                hipLaunchKernelGGL(k_repitch<true>, grid, dim3(256), 0, C.stream, C.stage_d, f.d(), C.L64, k0, rows);
+            } else {
+                hipLaunchKernelGGL(k_repitch<false>, grid, dim3(256), 0, C.stream, C.stage_d, f.d(), C.L64, k0, rows);
+                if ((rc = C.hip(hipMemcpyAsync(h, C.stage_d, bytes, hipMemcpyDeviceToHost, C.stream), "download"))) return rc;
+            }
+        }
+        return C.hip(hipStreamSynchronize(C.stream), "sync");
+    }
+    hipMemcpy3DParms p{};
+    const hipPitchedPtr hp = make_hipPitchedPtr(host, sizeof(double) * C.ng[0], C.ng[0], C.ng[1]);
+    const hipPitchedPtr dp = make_hipPitchedPtr(f.d() + C.L64.ox, sizeof(double) * C.L64.px, C.ng[0], C.ng[1]);
+    p.srcPtr = up ? hp : dp;
+    p.dstPtr = up ? dp : hp;
+    p.extent = make_hipExtent(sizeof(double) * C.ng[0], C.ng[1], C.ng[2]);
+    p.kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+    rc = C.hip(hipMemcpy3DAsync(&p, C.stream), up ? "upload" : "download");
+    if (rc) return rc;
+    return C.hip(hipStreamSynchronize(C.stream), "sync");
+}
+
 extern "C" {
 
 int pps_abi_version(void) { return PPS_ABI_VERSION; }
@@ -1519,6 +1611,7 @@ void pps_destroy(void* ctx)
         if (f.p) (void)hipFree(f.p);
     for (auto* p : C->flux_d)
         if (p) (void)hipFree(p);
+    if (C->stage_d) (void)hipFree(C->stage_d);
     if (C->rb.partials) (void)hipFree(C->rb.partials);
     if (C->rb.partials2) (void)hipFree(C->rb.partials2);
     if (C->rb.counter) (void)hipFree(C->rb.counter);
@@ -1542,49 +1635,18 @@ int pps_get_extent(void* ctx, int ng[3])
     return PPS_OK;
 }
 
-static int field_of(Ctx& C, int id, Field& f)
-{
-    if (id < 0 || id >= PPS_NUM_FIELDS) return C.fail(PPS_ERR_ARG, "bad field id %d", id);
-    if (!C.fields[id].p) {
-        int rc = C.alloc_field(C.fields[id], 64);
-        if (rc) return rc;
-    }
-    f = C.fields[id];
-    return PPS_OK;
-}
-
 int pps_upload(void* ctx, int field, const double* host)
 {
     Ctx* C = as_ctx(ctx);
     if (!C || !host) return PPS_ERR_ARG;
-    Field f;
-    int rc = field_of(*C, field, f);
-    if (rc) return rc;
-    hipMemcpy3DParms p{};
-    p.srcPtr = make_hipPitchedPtr(const_cast<double*>(host), sizeof(double) * C->ng[0], C->ng[0], C->ng[1]);
-    p.dstPtr = make_hipPitchedPtr(f.d() + C->L64.ox, sizeof(double) * C->L64.px, C->ng[0], C->ng[1]);
-    p.extent = make_hipExtent(sizeof(double) * C->ng[0], C->ng[1], C->ng[2]);
-    p.kind = hipMemcpyHostToDevice;
-    rc = C->hip(hipMemcpy3DAsync(&p, C->stream), "upload");
-    if (rc) return rc;
-    return C->hip(hipStreamSynchronize(C->stream), "sync");
+    return transfer(*C, field, const_cast<double*>(host), true);
 }
 
 int pps_download(void* ctx, int field, double* host)
 {
     Ctx* C = as_ctx(ctx);
     if (!C || !host) return PPS_ERR_ARG;
-    Field f;
-    int rc = field_of(*C, field, f);
-    if (rc) return rc;
-    hipMemcpy3DParms p{};
-    p.srcPtr = make_hipPitchedPtr(f.d() + C->L64.ox, sizeof(double) * C->L64.px, C->ng[0], C->ng[1]);
-    p.dstPtr = make_hipPitchedPtr(host, sizeof(double) * C->ng[0], C->ng[0], C->ng[1]);
-    p.extent = make_hipExtent(sizeof(double) * C->ng[0], C->ng[1], C->ng[2]);
-    p.kind = hipMemcpyDeviceToHost;
-    rc = C->hip(hipMemcpy3DAsync(&p, C->stream), "download");
-    if (rc) return rc;
-    return C->hip(hipStreamSynchronize(C->stream), "sync");
+    return transfer(*C, field, host, false);
 }
 
 int pps_fill(void* ctx, int field, double value)
