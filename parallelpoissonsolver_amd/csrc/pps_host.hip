@@ -280,8 +280,9 @@ static int scal_read(Ctx& C, const Scal* S, Scal& out)
 }
 
 // Runs `body` (one iteration's launches) until S->done, two batches in flight.
+// bodies_per_it: the most bodies that one iteration can take.
 template <class Body>
-static int run_loop(Ctx& C, Scal* S, int maxit, bool host_each, Body body)
+static int run_loop(Ctx& C, Scal* S, int maxit, bool host_each, Body body, int bodies_per_it = 1)
 {
     if (maxit <= 0) return PPS_OK;  // while (iter < maxIteration) never runs
     // Batch size: 4 doubling, then sized from the measured time per iteration
@@ -294,7 +295,7 @@ static int run_loop(Ctx& C, Scal* S, int maxit, bool host_each, Body body)
     constexpr double kBatchMs = 5.0;
     using clock = std::chrono::steady_clock;
     int batch = host_each ? 1 : 4;
-    int queued = 0;
+    long long queued = 0;
     int slot = 0;
     bool have_prev = false;
     int n_slot[2] = {0, 0};  // iterations of the batch behind each event
@@ -337,7 +338,7 @@ static int run_loop(Ctx& C, Scal* S, int maxit, bool host_each, Body body)
             else
                 batch = std::min(batch * 2, 64);
         }
-        if (queued > maxit + 2 * 64) break;  // every gate is closed by now
+        if (queued > (long long)bodies_per_it * maxit + 2 * 64) break;  // every gate is closed by now
     }
     return C.hip(hipStreamSynchronize(C.stream), "sync");
 }
@@ -606,7 +607,7 @@ struct KrylovStage : Stage {
         scale_box(C, b, S, 1);
     }
     // true-residual finish of a main solve (pps_stage::true_finish): r = b - A x
-    // of the complete x in FP64 (launch_residual modes 2-4); h->done tells
+    // of the complete x in FP64 (launch_residual modes 2, 3); h->done tells
     // whether the solve ends here
     int replace_residual(Field x, Field b, Field r, int mode, Scal* h)
     {
@@ -625,20 +626,23 @@ struct CGStage : KrylovStage {
     {
         if (prec() != 64 || x.prec != 64) return C.fail(PPS_ERR_UNSUPPORTED, "CG stage %d: FP32 vectors only inside PPS_IR", level);
         const std::string k = "cg" + std::to_string(level);
-        Field r, p0, p1, Ap, z;
+        double c = 1.0;
+        const bool pw = pre_pointwise(&c);
+        Field r, r2, p0, p1, Ap, z;
         int rc = C.get_work(k + ".r", 64, r);
         if (!rc) rc = C.get_work(k + ".p0", 64, p0);
         if (!rc) rc = C.get_work(k + ".p1", 64, p1);
-        if (!rc) rc = C.get_work(k + ".Ap", 64, Ap);
-        double c = 1.0;
-        const bool pw = pre_pointwise(&c);
+        if (!rc && pw) rc = C.get_work(k + ".r2", 64, r2);
+        if (!rc && !pw) rc = C.get_work(k + ".Ap", 64, Ap);
         if (!rc && !pw) rc = C.get_work(k + ".z", 64, z);
         if (rc) return rc;
         C.zero(r);
         C.zero(p0);
         C.zero(p1);
-        C.zero(Ap);
-        if (!pw) C.zero(z);
+        if (!pw) {
+            C.zero(Ap);
+            C.zero(z);
+        }
         rc = scal_init(C, S, cfg.tol, cfg.max_iter, pw ? c : 1.0, main ? C.hist_d : nullptr, main ? C.hist_cap : 0);
         if (rc) return rc;
         int early = 0;
@@ -651,11 +655,11 @@ struct CGStage : KrylovStage {
             if (rc) return rc;
             launch_cg_rz<double>(g, C.stream, C.rb, r.d(), z.d(), S);
         }
-        Field p[2] = {p0, p1};
+        Field p[2] = {p0, p1}, rr[2] = {r, r2};
         // where the device holds a ring of directions, x's updates are deferred
-        // to one pass per nring iterations (iteration q's direction in slot q
-        // mod nring; slot 0 = p1 and the last slot = p0 are zero, so the first
-        // iteration reads zeros as its old direction)
+        // to one pass per nring passes (pass q's direction in slot q mod nring;
+        // slot 0 = p1 and the last slot = p0 are zero, so the first pass reads
+        // zeros as its old direction)
         Field ring[kFcgRing];
         double* ringp[kFcgRing] = {};
         int nring = 0;
@@ -663,29 +667,22 @@ struct CGStage : KrylovStage {
         if (rc) return rc;
         for (int j = 0; j < nring; ++j) ringp[j] = ring[j].d();
         if (nring) launch_fcg_ring_reset(C.stream, S);
-        int q = 0;
-        int cur = 0;
+        int q = 0;  // passes queued: pass q reads p[q & 1] (and rr[q & 1]) and writes the other one
         auto body = [&]() -> int {
-            // iteration k reads p[k&1], writes p[(k+1)&1], and applies
-            // iteration k-1's x update on the way (with the ring: reads slot
-            // k-1, writes slot k, and leaves x to the flush)
-            if (nring) {
-                const int qs = q % nring, qo = (q + nring - 1) % nring;
-                launch_cg_A2<double>(g, C.stream, C.rb, pw ? r.d() : z.d(), ring[qo].d(), ring[qs].d(), Ap.d(), x.d(),
-                                     S, pw, qs);
-                if (qs == nring - 1) launch_fcg_flush<double>(g, C.stream, x.d(), ringp, S);
-                ++q;
-            } else {
-                launch_cg_A2<double>(g, C.stream, C.rb, pw ? r.d() : z.d(), p[cur].d(), p[cur ^ 1].d(), Ap.d(), x.d(), S,
-                                     pw);
-            }
-            cur ^= 1;
-            launch_cg_B<double>(g, C.stream, C.rb, r.d(), Ap.d(), S, pw, main);
-            if (!pw) {
-                int e = pre_apply(z, r, &S->done);
-                if (e) return e;
-                launch_cg_rz<double>(g, C.stream, C.rb, r.d(), z.d(), S);
-            }
+            // pass q also applies pass q - 1's x update (with the ring: reads
+            // slot q - 1, writes slot q, and leaves x to the flush)
+            const int cur = q & 1, qs = nring ? q % nring : -1, qo = nring ? (q + nring - 1) % nring : 0;
+            const double* pin = nring ? ring[qo].d() : p[cur].d();
+            double* pout = nring ? ring[qs].d() : p[cur ^ 1].d();
+            if (pw) launch_cg_pass<double>(g, C.stream, C.rb, rr[cur].d(), pin, rr[cur ^ 1].d(), pout, x.d(), S, main, qs);
+            else launch_cg_A2<double>(g, C.stream, C.rb, z.d(), pin, pout, Ap.d(), x.d(), S, qs);
+            if (nring && qs == nring - 1) launch_fcg_flush<double>(g, C.stream, x.d(), ringp, S);
+            ++q;
+            if (pw) return PPS_OK;
+            launch_cg_B<double>(g, C.stream, C.rb, r.d(), Ap.d(), S, main);
+            int e = pre_apply(z, r, &S->done);
+            if (e) return e;
+            launch_cg_rz<double>(g, C.stream, C.rb, r.d(), z.d(), S);
             return PPS_OK;
         };
         Scal h;
@@ -694,19 +691,21 @@ struct CGStage : KrylovStage {
         long long pre_calls = pw ? 0 : 1;
         int it0 = 0;
         for (int repl = 0;; ++repl) {
-            rc = run_loop(C, S, cfg.max_iter, pre_host(), body);
+            // a pass may recompute the residual instead of iterating
+            rc = run_loop(C, S, cfg.max_iter, pre_host(), body, pw ? 2 : 1);
             if (rc) return rc;
-            // the last executed iteration K-1 left x += alpha_{K-1} p_{K-1} pending; p_{K-1} is p[K&1]
+            // the last pass that ran, n - 1, left x += alpha p pending; its direction is p[n & 1]
             rc = scal_read(C, S, h);
             if (rc) return rc;
             if (!pw) pre_calls += std::max(0, h.iter - it0 - 1);
             it0 = h.iter;
+            const int n = pw ? h.passes : h.iter;
             if (nring) launch_fcg_flush<double>(g, C.stream, x.d(), ringp, S);
-            else if (h.iter > 0) launch_cg_final_x<double>(g, C.stream, x.d(), p[h.iter & 1].d(), S);
+            else if (n > 0) launch_cg_final_x<double>(g, C.stream, x.d(), p[n & 1].d(), S);
             if (!main || repl >= cfg.true_finish) break;
-            // true-residual finish: r = b - A x of the complete x replaces the
-            // recursive residual; the search direction p[K&1] and beta stay
-            rc = replace_residual(x, b, r, pw ? 3 : 2, &h);
+            // true-residual finish: r = b - A x of the complete x, written where
+            // the next pass reads its residual; the search direction and beta stay
+            rc = replace_residual(x, b, pw ? rr[n & 1] : r, 2, &h);
             if (rc) return rc;
             if (h.done) break;
             if (!pw) {
@@ -715,8 +714,7 @@ struct CGStage : KrylovStage {
                 launch_cg_rz<double>(g, C.stream, C.rb, r.d(), z.d(), S);
                 ++pre_calls;
             }
-            cur = h.iter & 1;
-            q = h.iter;  // queued iterations past the stop advanced q without running
+            q = n;  // passes queued past the stop advanced q without running
         }
         count_pre(pre_calls);
         epilogue(main, x, b, r);
@@ -801,7 +799,7 @@ struct BiCGStage : KrylovStage {
             if (!main || repl >= cfg.true_finish) break;
             // true-residual finish: restart from r = b - A x with r0 = p = r
             Scal h;
-            rc = replace_residual(x, b, r, 4, &h);
+            rc = replace_residual(x, b, r, 3, &h);
             if (rc) return rc;
             if (h.done) break;
             launch_copy<double>(g, C.stream, r.d(), p.d());
@@ -1089,20 +1087,21 @@ struct IRStage : KrylovStage {
         Field p0, p1, A0, A1, z;
         int rc = C.get_work(k + ".p0", 32, p0);
         if (!rc) rc = C.get_work(k + ".p1", 32, p1);
-        if (!rc) rc = C.get_work(k + ".A0", 32, A0);
-        if (!rc) rc = C.get_work(k + ".A1", 32, A1);
-        if (rc) return rc;
         Stage* M = in->pre;
         double c = 1.0;
         const bool pw = (M == nullptr) || M->pointwise(&c);
         const bool flexible = in->cfg.kind == PPS_FCG;
+        const bool one_pass = !flexible && pw;  // CG with a pointwise preconditioner
+        if (!rc && !one_pass) rc = C.get_work(k + ".A0", 32, A0);
+        if (!rc && !one_pass) rc = C.get_work(k + ".A1", 32, A1);
+        if (rc) return rc;
         if ((!pw || flexible) && (rc = C.get_work(k + ".z", 32, z))) return rc;
         // FCG with a preconditioner that forms the residual update itself (the
         // learned one): r alternates between r32 and a second field, written by
         // the preconditioner, and the update pass drops out of the loop
         const bool fused_r = flexible && M && M->forms_update();
         Field rr[2] = {r32, r32};
-        if (fused_r && (rc = C.get_work(k + ".r32b", 32, rr[1]))) return rc;
+        if ((fused_r || one_pass) && (rc = C.get_work(k + ".r32b", 32, rr[1]))) return rc;
         // SI was initialised by solve_main; the outer residual kernel has just
         // written SI[S_INNER_NORM], and ir_inner_init resets iter/done
         const Geo g = C.gsolver(32);
@@ -1121,13 +1120,15 @@ struct IRStage : KrylovStage {
             if (rc) return rc;
             for (int j = 0; j < nring; ++j) ringp[j] = ring[j].f();
         }
-        launch_ir_inner_init(g, C.stream, C.rb, r32.f(), d.f(), p0.f(), SI, pw);
+        launch_ir_inner_init(g, C.stream, C.rb, r32.f(), d.f(), p0.f(), SI);
         if (nring) launch_fcg_ring_reset(C.stream, SI);
         int q = 0;
         // pin p1 and the old Ap to zero as well: iteration 0 multiplies them by beta = 0
         launch_fill<float>(g, C.stream, p1.f(), 0.0f);
-        launch_fill<float>(g, C.stream, A0.f(), 0.0f);
-        launch_fill<float>(g, C.stream, A1.f(), 0.0f);
+        if (!one_pass) {
+            launch_fill<float>(g, C.stream, A0.f(), 0.0f);
+            launch_fill<float>(g, C.stream, A1.f(), 0.0f);
+        }
         int cur = 0;
         const bool host_each = M && M->host_driven();
         auto applyM = [&](const int* gate) -> int {
@@ -1176,32 +1177,30 @@ struct IRStage : KrylovStage {
                 launch_fcg_update<float>(g, C.stream, C.rb, r32.f(), Ap[cur].f(), SI, false);
                 cur ^= 1;
             } else {
-                if (nring) {
-                    const int qs = q % nring, qo = (q + nring - 1) % nring;
-                    launch_cg_A2<float>(g, C.stream, C.rb, pw ? r32.f() : z.f(), ring[qo].f(), ring[qs].f(), Ap[0].f(),
-                                        d.f(), SI, pw, qs);
-                    if (qs == nring - 1) launch_fcg_flush<float>(g, C.stream, d.f(), ringp, SI);
-                    ++q;
-                } else {
-                    launch_cg_A2<float>(g, C.stream, C.rb, pw ? r32.f() : z.f(), p[cur].f(), p[cur ^ 1].f(), Ap[0].f(),
-                                        d.f(), SI, pw);
-                }
+                const int qs = nring ? q % nring : -1, qo = nring ? (q + nring - 1) % nring : 0;
+                const float* pin = nring ? ring[qo].f() : p[cur].f();
+                float* pout = nring ? ring[qs].f() : p[cur ^ 1].f();
+                if (one_pass) launch_cg_pass<float>(g, C.stream, C.rb, rr[cur].f(), pin, rr[cur ^ 1].f(), pout, d.f(), SI, false, qs);
+                else launch_cg_A2<float>(g, C.stream, C.rb, z.f(), pin, pout, Ap[0].f(), d.f(), SI, qs);
+                if (nring && qs == nring - 1) launch_fcg_flush<float>(g, C.stream, d.f(), ringp, SI);
+                ++q;
                 cur ^= 1;
-                launch_cg_B<float>(g, C.stream, C.rb, r32.f(), Ap[0].f(), SI, pw, false);
-                if (!pw) {
+                if (!one_pass) {
+                    launch_cg_B<float>(g, C.stream, C.rb, r32.f(), Ap[0].f(), SI, false);
                     int e = applyM(&SI->done);
                     if (e) return e;
                     launch_cg_rz<float>(g, C.stream, C.rb, r32.f(), z.f(), SI);
                 }
             }
             return PPS_OK;
-        });
+        }, one_pass ? 2 : 1);
         if (rc) return rc;
         Scal h;
         rc = scal_read(C, SI, h);
         if (rc) return rc;
         if (nring) launch_fcg_flush<float>(g, C.stream, d.f(), ringp, SI);  // the ring's last steps
-        else if (!flexible && h.iter > 0) launch_cg_final_x<float>(g, C.stream, d.f(), p[h.iter & 1].f(), SI);
+        else if (!flexible && h.iter > 0)
+            launch_cg_final_x<float>(g, C.stream, d.f(), p[(one_pass ? h.passes : h.iter) & 1].f(), SI);
         else if (flexible && h.iter > 0) launch_fcg_final_x<float>(g, C.stream, d.f(), p[(h.iter - 1) & 1].f(), SI);
         inner_total += h.iter;
         if (flexible) C.fallback_switches += h.fallback;
@@ -1549,7 +1548,9 @@ int pps_create(const pps_grid* grid, void** out)
     // the span sums of the two-level epilogue
     const Geo gbig = make_geo(X.L64, X.box, X.coef, kMinKz, 0);
     const long long nvec = (long long)((X.ng[0] + kThreads - 1) / kThreads) * X.ng[1] * X.ng[2];
-    X.rb.cap = (int)std::max<long long>(gbig.nblocks, nvec) + 8;
+    // one-plane chunks of 64 x 16 tiles (small grids' CG pass)
+    const long long nsmall = (long long)((X.ng[0] + kTX - 1) / kTX) * ((X.ng[1] + 15) / 16) * X.ng[2];
+    X.rb.cap = (int)std::max(std::max<long long>(gbig.nblocks, nvec), nsmall) + 8;
     X.rb.cap2 = X.rb.cap / kSpan + 8;
     rc = rc ? rc : X.hip(hipMalloc(&X.rb.partials2, sizeof(double) * kMaxRedQ * X.rb.cap2), "span partials");
     // a solve streams 4-8 fields per iteration: once a field passes 32 MiB
@@ -2054,14 +2055,14 @@ int pps_time_kernel(void* ctx, int kernel, int reps, double* ms, double* bytes)
         switch (kernel) {
         case PPS_K_CG_STENCIL:
             launch_cg_A2<double>(g, C->stream, C->rb, a.d(), (it & 1) ? c.d() : b.d(), (it & 1) ? b.d() : c.d(), d.d(),
-                                 e.d(), S, true, 0);
+                                 e.d(), S, 0);
             break;
         case PPS_K_CG_STENCIL_F32:
             launch_cg_A2<float>(g, C->stream, C->rb, a.f(), (it & 1) ? c.f() : b.f(), (it & 1) ? b.f() : c.f(), d.f(),
-                                e.f(), S, true, 0);
+                                e.f(), S, 0);
             break;
-        case PPS_K_CG_UPDATE: launch_cg_B<double>(g, C->stream, C->rb, a.d(), c.d(), S, true, false); break;
-        case PPS_K_CG_UPDATE_F32: launch_cg_B<float>(g, C->stream, C->rb, a.f(), c.f(), S, true, false); break;
+        case PPS_K_CG_UPDATE: launch_cg_B<double>(g, C->stream, C->rb, a.d(), c.d(), S, false); break;
+        case PPS_K_CG_UPDATE_F32: launch_cg_B<float>(g, C->stream, C->rb, a.f(), c.f(), S, false); break;
         case PPS_K_RESIDUAL: launch_residual(g, C->stream, C->rb, a.d(), b.d(), c.d(), S, 1); break;
         case PPS_K_COPY: launch_copy<double>(g, C->stream, a.d(), e.d()); break;
         case PPS_K_CHEB_SWEEP: launch_cheb_sweep<double, double>(g, C->stream, a.d(), b.d(), c.d(), e.d(), 0.1, 0.2, 0.3, 1.0, nullptr); break;
@@ -2350,6 +2351,9 @@ int pps_nn_generate(void* nn, const pps_nn_train_cfg* cfg, long long* pairs)
     }
     std::unique_ptr<void, void (*)(void*)> guard(cx, pps_destroy);
     Ctx* C = as_ctx(cx);
+    // a fixed z-chunk: the sums' order, and with it the pairs' last bits (which
+    // training amplifies), then do not follow the launch tuning
+    C->kz_st = 4;
     // scratch fields are allocated on first use: the raw kernels below write T1/T2
     for (int id : {PPS_FIELD_T0, PPS_FIELD_T1, PPS_FIELD_T2, PPS_FIELD_T3}) {
         Field f;

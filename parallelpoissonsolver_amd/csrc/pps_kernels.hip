@@ -750,8 +750,7 @@ struct OpResidual : Gate {
     double* __restrict__ r;
     Scal* S;
     int mode;
-    double jac;
-    __device__ void load() { jac = S->v[S_JAC]; }
+    __device__ void load() {}
     struct Ox { double b; };
     __device__ double in(long long c) const { return x[c]; }
     template <bool NT> __device__ Ox out_raw(long long c) const { return {ld<NT>(b + c)}; }
@@ -760,7 +759,6 @@ struct OpResidual : Gate {
         const double rv = o.b - Av;
         put<NT>(r + c, rv);
         acc[0] += rv * rv;
-        acc[1] += rv * (jac * rv);
     }
     __device__ void finish(const double* t)
     {
@@ -769,7 +767,6 @@ struct OpResidual : Gate {
             S->v[S_ERR0] = e;
             S->v[S_ERR] = e;
             S->v[S_ERR_OP] = e;
-            S->v[S_RZ] = t[1];
             S->v[S_RR] = t[0];
             S->v[S_BETA] = 0.0;
             S->v[S_RHO0] = 1.0;
@@ -786,8 +783,7 @@ struct OpResidual : Gate {
             S->v[S_ERR_OP] = e;
             S->v[S_RR] = t[0];
             S->v[S_ALPHA] = 0.0;  // x is complete: no pending update
-            if (mode == 3) S->v[S_RZ] = t[1];   // CG, pointwise preconditioner: r.(jac r) of the new r
-            if (mode == 4) S->v[S_RHO0] = t[0]; // BiCGSTAB restarted with r0 = r: rho = r0.r
+            if (mode == 3) S->v[S_RHO0] = t[0]; // BiCGSTAB restarted with r0 = r: rho = r0.r
             S->done = (e < S->v[S_TOL] || S->iter >= S->maxit) ? 1 : 0;
         }
     }
@@ -802,7 +798,7 @@ void launch_residual(const Geo& g, hipStream_t s, RedBuf rb, const double* x, co
     op.r = r;
     op.S = S;
     op.mode = mode;
-    run_stencil<double, 2>(g, s, op, rb);
+    run_stencil<double, 1>(g, s, op, rb);
 }
 
 // r = b - A x and ||r|| into one device double: the residual above without a
@@ -999,10 +995,333 @@ void launch_ghost(hipStream_t s, const Layout& L, const Faces& F, T* field, int 
 
 // ------------------------------------------------------------------- CG
 
-// p_new = a*src + beta*p_old, Ap = A p_new, p.Ap ; alpha = rz / pAp  (baseCG.hpp:126-150,197-207)
-// The reference updates x and r together after alpha is known (baseCG.hpp:154-165);
-// here x's update for iteration k-1 rides along with iteration k's stencil
-// pass, which reads p_{k-1} anyway: the same x after every iteration, one
+// One CG iteration in one pass over the grid (pointwise preconditioner M = jac I;
+// baseCG.hpp:126-207 has two reductions and a pass for each):
+//   r = r_old - alpha_old A p_old      the previous iteration's update
+//   p = jac r + beta p_old             the new direction
+//   sums r.r, p.Ap, r.Ap, Ap.Ap        finish: alpha = jac r.r / p.Ap and
+//   ||r - alpha Ap||^2 = r.r - 2 alpha r.Ap + alpha^2 Ap.Ap, hence beta and the
+//   convergence test, before the next residual has been formed.
+// A p_old is recomputed from p_old instead of being stored, so a pass reads
+// r_old and p_old and writes r and p: 4 words per point and iteration where a
+// stencil pass plus an update pass move 7.  r.r is summed from the residual
+// itself in every pass; the expansion only predicts the next one.  It loses
+// digits when one step removes most of r: below kCgRecheck r.r the next pass
+// only forms r (p is kept, no iteration is counted) and beta and the
+// convergence test take its sum.
+//
+// Measured at 512^3 FP64: 0.85 ms for its 4 words (5.06 TB/s; 5.4 with the rings'
+// re-reads that miss L2, 1.14x on the reads), where the stencil and update
+// passes took 0.83 + 0.53 ms; 1.10 against 1.60 ms per iteration with x's
+// deferred updates.  The HBM rate is that of the other marching stencils.
+//
+// A block owns a 64 x (8 RY) tile and marches z.  It forms p on the tile and a
+// one-point ring, from p_old on the tile and a two-point ring; a thread owns RY
+// consecutive rows of one column (their y-neighbours are its own registers)
+// and at most one point of each ring.  Per plane: p_old of plane s goes to
+// LDS, one barrier, then p of plane s (to the other LDS array) and A p of plane
+// s - 1, whose neighbours went to LDS one plane earlier.  Both arrays alternate
+// between two planes, so one barrier separates every write from its readers:
+// p_old's buffer is rewritten two steps later, after the barrier that all its
+// readers have passed, and p of plane s - 1 was written before this plane's
+// barrier.  Every rounding is spelled out (explicit fma, or none) so that a ring
+// point and the tile point it mirrors in the neighbouring block round alike.
+constexpr double kCgRecheck = 1e-2;  // beta's relative error stays near eps / kCgRecheck
+constexpr int kCgW = 8;              // wavefronts per block
+
+template <typename T>
+__device__ __forceinline__ T lap7(T v, T xm, T xp, T ym, T yp, T zm, T zp, T cx, T cy, T cz)
+{
+    const T dx = (xm - v) + (xp - v), dy = (ym - v) + (yp - v), dz = (zm - v) + (zp - v);
+    return fma(cx, dx, fma(cy, dy, cz * dz));
+}
+
+// p = z + beta p_old with z = jac r, each product rounded, as the reference
+// forms it (baseCG.hpp:139,199-203)
+template <typename T>
+__device__ __forceinline__ T cg_direction(T r, T p_old, T jac, T beta)
+{
+#pragma clang fp contract(off)
+    const T z = jac * r, bp = beta * p_old;
+    return z + bp;
+}
+
+template <typename T>
+struct CgPassArgs {
+    const T* __restrict__ r_in;
+    const T* __restrict__ pin;
+    T* __restrict__ r_out;
+    T* __restrict__ pout;
+    T* __restrict__ x;  // null: x's updates are deferred to the ring's flush
+    const Scal* S;
+};
+
+// point t of the ring around a box of W x H points -> (row, col) in the box's frame
+template <int W, int H>
+__device__ __forceinline__ void ring_point(int t, int& r, int& c)
+{
+    if (t < W + 2) { r = -1; c = t - 1; }
+    else if (t < 2 * (W + 2)) { r = H; c = t - (W + 2) - 1; }
+    else if (t < 2 * (W + 2) + H) { r = t - 2 * (W + 2); c = -1; }
+    else { r = t - 2 * (W + 2) - H; c = W; }
+}
+
+template <typename T, int RY, bool XUPD, bool NT>
+__global__ __launch_bounds__(kTX* kCgW) void k_cg_pass(Geo g, CgPassArgs<T> A, RedBuf rb)
+{
+    if (A.S->done) return;
+    constexpr int TY = kCgW * RY;
+    constexpr int N1 = 2 * (kTX + 2) + 2 * TY, N2 = 2 * (kTX + 4) + 2 * (TY + 2);
+    static_assert(N1 <= kTX * kCgW && N2 <= kTX * kCgW, "ring points need one thread each");
+    __shared__ T ysl[2][TY + 4][kTX + 4];  // p_old, tile and two-point ring
+    __shared__ T wsl[2][TY + 2][kTX + 2];  // p, tile and one-point ring
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int tx0 = b % g.ntx, rr = b / g.ntx;
+    const int ty0 = rr % g.nty, tz0 = rr / g.nty;
+    const int i0 = g.lo0 + tx0 * kTX, j0 = g.lo1 + ty0 * TY;
+    const int k0 = g.lo2 + tz0 * g.kz, k1 = min(k0 + g.kz, g.hi2);
+    const int lx = threadIdx.x, ly = threadIdx.y, tid = lx + kTX * ly;
+    const T cx = (T)g.cx, cy = (T)g.cy, cz = (T)g.cz;
+    const bool recheck = A.S->recheck != 0;
+    const T alpha = (T)A.S->v[S_ALPHA];
+    const T beta = recheck ? T(1) : (T)A.S->v[S_BETA];
+    const T jac = recheck ? T(0) : (T)A.S->v[S_JAC];
+
+    // points of this thread: RY tile rows, one point of each ring; a point off
+    // the solver region holds 0 and is never loaded
+    const long long px = g.px;
+    const long long t0 = (long long)g.ox + (i0 + lx) + px * (j0 + ly * RY);
+    bool in[RY];
+#pragma unroll
+    for (int q = 0; q < RY; ++q) in[q] = i0 + lx < g.hi0 && j0 + ly * RY + q < g.hi1;
+    int r1 = 0, c1 = 0, r2 = 0, c2 = 0;
+    const bool has1 = tid < N1, has2 = tid < N2;
+    if (has1) ring_point<kTX, TY>(tid, r1, c1);
+    if (has2) {
+        ring_point<kTX + 2, TY + 2>(tid, r2, c2);
+        r2 -= 1;
+        c2 -= 1;
+    }
+    auto inxy = [&](int i, int j) { return i >= g.lo0 && i < g.hi0 && j >= g.lo1 && j < g.hi1; };
+    const bool in1 = has1 && inxy(i0 + c1, j0 + r1), in2 = has2 && inxy(i0 + c2, j0 + r2);
+    const long long o1 = (long long)g.ox + (i0 + c1) + px * (j0 + r1);
+    const long long o2 = (long long)g.ox + (i0 + c2) + px * (j0 + r2);
+
+    T pm[RY], pc[RY], pp[RY], pn[RY], rc[RY], rn[RY], rv[RY], wm[RY], wc[RY], wn[RY], xc[RY], xn[RY];
+    T qm = 0, qc = 0, qp = 0, qn = 0, qr = 0, qrn = 0, oc = 0, on = 0;
+    auto zin = [&](int k) { return k >= g.lo2 && k < g.hi2; };
+    const int s0 = k0 - 1;
+    {
+        const bool za = zin(s0 - 1), zb = zin(s0), zc = zin(s0 + 1);
+        const long long fa = g.plane * (s0 - 1), fb = g.plane * s0, fc = g.plane * (s0 + 1);
+#pragma unroll
+        for (int q = 0; q < RY; ++q) {
+            pm[q] = in[q] && za ? A.pin[t0 + px * q + fa] : T(0);
+            pc[q] = in[q] && zb ? A.pin[t0 + px * q + fb] : T(0);
+            pp[q] = in[q] && zc ? A.pin[t0 + px * q + fc] : T(0);
+            rc[q] = in[q] && zb ? A.r_in[t0 + px * q + fb] : T(0);
+            pn[q] = rn[q] = rv[q] = wm[q] = wc[q] = wn[q] = xc[q] = xn[q] = T(0);
+        }
+        if (in1) {
+            qm = za ? A.pin[o1 + fa] : T(0);
+            qc = zb ? A.pin[o1 + fb] : T(0);
+            qp = zc ? A.pin[o1 + fc] : T(0);
+            qr = zb ? A.r_in[o1 + fb] : T(0);
+        }
+        if (in2 && zb) oc = A.pin[o2 + fb];
+    }
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int s = s0; s <= k1; ++s) {
+        const int buf = s & 1;
+        const long long fs = g.plane * s;
+#pragma unroll
+        for (int q = 0; q < RY; ++q) ysl[buf][ly * RY + q + 2][lx + 2] = pc[q];
+        if (has1) ysl[buf][r1 + 2][c1 + 2] = qc;
+        if (has2) ysl[buf][r2 + 2][c2 + 2] = oc;
+        // loads for the next step: p_old of plane s + 2 (s + 1 on the outer ring), r_old (and x) of plane s + 1
+        const bool z1 = s < k1 && zin(s + 1), z2 = s < k1 && zin(s + 2);
+        const long long f1 = fs + g.plane, f2 = f1 + g.plane;
+#pragma unroll
+        for (int q = 0; q < RY; ++q) {
+            pn[q] = in[q] && z2 ? A.pin[t0 + px * q + f2] : T(0);
+            rn[q] = in[q] && z1 ? A.r_in[t0 + px * q + f1] : T(0);
+            if constexpr (XUPD) xn[q] = in[q] && z1 && s + 1 < k1 ? ld<NT>(A.x + t0 + px * q + f1) : T(0);
+        }
+        if (in1) {
+            qn = z2 ? A.pin[o1 + f2] : T(0);
+            qrn = z1 ? A.r_in[o1 + f1] : T(0);
+        }
+        if (in2) on = z1 ? A.pin[o2 + f1] : T(0);
+        __syncthreads();
+        const bool zs = zin(s), own = s >= k0 && s < k1;
+        T rs[RY];
+#pragma unroll
+        for (int q = 0; q < RY; ++q) {
+            const int r = ly * RY + q + 2, c = lx + 2;
+            T w = T(0), v = T(0);
+            if (in[q] && zs) {
+                const T ym = q > 0 ? pc[q > 0 ? q - 1 : 0] : ysl[buf][r - 1][c];
+                const T yp = q + 1 < RY ? pc[q + 1 < RY ? q + 1 : 0] : ysl[buf][r + 1][c];
+                const T Ap = lap7(pc[q], ysl[buf][r][c - 1], ysl[buf][r][c + 1], ym, yp, pm[q], pp[q], cx, cy, cz);
+                v = fma(-alpha, Ap, rc[q]);
+                w = cg_direction(v, pc[q], jac, beta);
+                if (own) {
+                    put<NT>(A.r_out + t0 + px * q + fs, v);
+                    put<NT>(A.pout + t0 + px * q + fs, w);
+                    if constexpr (XUPD) put<NT>(A.x + t0 + px * q + fs, fma(alpha, pc[q], xc[q]));
+                    acc[0] += (double)v * (double)v;
+                }
+            }
+            rs[q] = v;
+            wn[q] = w;
+            wsl[buf][r - 1][c - 1] = w;
+        }
+        if (has1) {
+            T w = T(0);
+            if (in1 && zs) {
+                const int r = r1 + 2, c = c1 + 2;
+                const T Ap = lap7(qc, ysl[buf][r][c - 1], ysl[buf][r][c + 1], ysl[buf][r - 1][c], ysl[buf][r + 1][c], qm,
+                                  qp, cx, cy, cz);
+                w = cg_direction(fma(-alpha, Ap, qr), qc, jac, beta);
+            }
+            wsl[buf][r1 + 1][c1 + 1] = w;
+        }
+        // A p of plane s - 1
+        if (s > k0) {
+            const int pb = buf ^ 1;
+#pragma unroll
+            for (int q = 0; q < RY; ++q) {
+                if (!in[q]) continue;
+                const int r = ly * RY + q + 1, c = lx + 1;
+                const T ym = q > 0 ? wc[q > 0 ? q - 1 : 0] : wsl[pb][r - 1][c];
+                const T yp = q + 1 < RY ? wc[q + 1 < RY ? q + 1 : 0] : wsl[pb][r + 1][c];
+                const double Ap = (double)lap7(wc[q], wsl[pb][r][c - 1], wsl[pb][r][c + 1], ym, yp, wm[q], wn[q], cx, cy, cz);
+                acc[1] += (double)wc[q] * Ap;
+                acc[2] += (double)rv[q] * Ap;
+                acc[3] += Ap * Ap;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < RY; ++q) {
+            pm[q] = pc[q];
+            pc[q] = pp[q];
+            pp[q] = pn[q];
+            rc[q] = rn[q];
+            rv[q] = rs[q];
+            wm[q] = wc[q];
+            wc[q] = wn[q];
+            xc[q] = xn[q];
+        }
+        qm = qc;
+        qc = qp;
+        qp = qn;
+        qr = qrn;
+        oc = on;
+    }
+    block_partials<4, kTX * kCgW>(acc, rb, (int)blockIdx.x);
+}
+
+struct OpCgPass {
+    Scal* S;
+    bool history;
+    int slot;
+    __device__ __forceinline__ bool gated() const { return S->done != 0; }
+    __device__ void end_iteration(int it, double rr) const
+    {
+        const double err = sqrt(rr);
+        S->v[S_RR] = rr;
+        S->v[S_ERR] = err;
+        if (history && S->hist != nullptr && it < S->hist_cap) S->hist[it] = err;
+        if (err < S->v[S_TOL] || it >= S->maxit) S->done = 1;
+    }
+    __device__ void finish(const double* t) const
+    {
+        const double rr = t[0];
+        S->passes += 1;
+        if (S->recheck) {
+            // the pass formed r (x has its step already) and kept p
+            S->recheck = 0;
+            S->v[S_BETA] = rr / S->v[S_RR];
+            S->v[S_ALPHA] = 0.0;
+            if (slot >= 0) S->ahist[slot] = 0.0;
+            end_iteration(S->iter, rr);
+            return;
+        }
+        const double rz = S->v[S_JAC] * rr, a = rz / t[1];
+        S->v[S_RZ] = rz;
+        S->v[S_PAP] = t[1];
+        S->v[S_ALPHA] = a;
+        if (slot >= 0) S->ahist[slot] = a;
+        S->iter += 1;
+        const double next = rr - 2.0 * a * t[2] + a * a * t[3];
+        if (next > kCgRecheck * rr) {
+            S->v[S_BETA] = next / rr;
+            end_iteration(S->iter, next);
+        } else {
+            S->v[S_RR] = rr;
+            S->recheck = 1;
+        }
+    }
+};
+
+// z-chunk of a marching kernel whose blocks load `extra` planes beyond their
+// own and of which `slots` run at once: the one with the least work in the
+// busiest slot, ceil(blocks / slots) * (kz + extra) planes (the longest of
+// equals, up to 128 planes)
+static int pick_kz(long long tiles, int nz, int slots, int extra)
+{
+    int best = 1;
+    long long cost = -1;
+    for (int kz = 1; kz <= 128; ++kz) {
+        if (kz > 1 && kz > nz) break;
+        const long long nb = tiles * ((nz + kz - 1) / kz);
+        const long long c = ((nb + slots - 1) / slots) * (std::min(kz, nz) + extra);
+        if (cost < 0 || c <= cost) {
+            cost = c;
+            best = kz;
+        }
+    }
+    return best;
+}
+
+constexpr int kCUs = 256;  // compute units of the MI355X
+
+template <typename T, int RY>
+static void run_cg_pass(const Geo& g, hipStream_t s, const CgPassArgs<T>& A, const OpCgPass& op, RedBuf rb)
+{
+    if (!check_capacity<4, OpCgPass>(g, rb)) return;
+    const dim3 grid(g.nblocks), block(kTX, kCgW);
+    if (g.nt && A.x) hipLaunchKernelGGL((k_cg_pass<T, RY, true, true>), grid, block, 0, s, g, A, rb);
+    else if (g.nt) hipLaunchKernelGGL((k_cg_pass<T, RY, false, true>), grid, block, 0, s, g, A, rb);
+    else if (A.x) hipLaunchKernelGGL((k_cg_pass<T, RY, true, false>), grid, block, 0, s, g, A, rb);
+    else hipLaunchKernelGGL((k_cg_pass<T, RY, false, false>), grid, block, 0, s, g, A, rb);
+    launch_finish<4>(s, op, rb, g.nblocks);
+}
+
+template <typename T>
+void launch_cg_pass(const Geo& g0, hipStream_t s, RedBuf rb, const T* r_in, const T* pin, T* r_out, T* pout, T* x,
+                    Scal* S, bool history, int ring_slot)
+{
+    const CgPassArgs<T> A{r_in, pin, r_out, pout, ring_slot < 0 ? x : nullptr, S};
+    const OpCgPass op{S, history, ring_slot};
+    const int nx = g0.hi0 - g0.lo0, ny = g0.hi1 - g0.lo1, nz = g0.hi2 - g0.lo2;
+    if (nx <= 0 || ny <= 0 || nz <= 0) return;
+    auto tiles = [&](int th) { return (long long)((nx + kTX - 1) / kTX) * ((ny + th - 1) / th); };
+    auto tiling = [&](int th, int slots) {
+        return retile(g0, th, g0.kz_st > 0 ? g0.kz_st : pick_kz(tiles(th), nz, slots, 4));
+    };
+    // 32-row tiles (one block per CU: 158 VGPRs) read fewer ring points and win
+    // where there is enough work for two 16-plane chunks per CU, 16-row tiles (two
+    // blocks per CU) below that.  us per iteration, 32 / 16 rows, FP64: 514^3
+    // 1110 / 1169, 258^3 145 / 148, 194^3 77.5 / 71.5, 130^3 32.8 / 27.1, 66^3 15.5 / 13.9
+    if (tiles(4 * kCgW) * nz >= 2ll * 16 * kCUs) run_cg_pass<T, 4>(tiling(4 * kCgW, kCUs), s, A, op, rb);
+    else run_cg_pass<T, 2>(tiling(2 * kCgW, 2 * kCUs), s, A, op, rb);
+}
+
+// buffer-preconditioned CG: p_new = z + beta*p_old, Ap = A p_new, p.Ap ; alpha = rz / pAp
+// (baseCG.hpp:126-150,197-207).  The reference updates x and r together after alpha is
+// known (baseCG.hpp:154-165); here x's update for iteration k-1 rides along with iteration
+// k's stencil pass, which reads p_{k-1} anyway: the same x after every iteration, one
 // fewer field pass per iteration.  The last update runs after the loop.
 template <typename T>
 struct OpCgA : Gate {
@@ -1012,19 +1331,17 @@ struct OpCgA : Gate {
     T* __restrict__ Ap;
     T* __restrict__ x;
     Scal* S;
-    bool pointwise;
     int slot;  // >= 0: deferred x updates (x untouched; alpha to S->ahist[slot])
-    T a, beta, alpha_prev;
+    T beta, alpha_prev;
     __device__ void load()
     {
-        a = pointwise ? (T)S->v[S_JAC] : T(1);
         beta = (T)S->v[S_BETA];
         alpha_prev = (T)S->v[S_ALPHA];
     }
     struct Raw { T src, pold; };  // p_old at the point also feeds the folded x update
     struct Ox { T x; };
     __device__ Raw in_raw(long long c) const { return {src[c], pin[c]}; }
-    __device__ T in_value(const Raw& r) const { return a * r.src + beta * r.pold; }
+    __device__ T in_value(const Raw& r) const { return r.src + beta * r.pold; }
     template <bool NT> __device__ Ox out_raw(long long c) const { return {slot < 0 ? ld<NT>(x + c) : T(0)}; }
     template <bool NT> __device__ void out(long long c, T vc, T Av, const Raw& r, const Ox& o, double* acc) const
     {
@@ -1044,18 +1361,17 @@ struct OpCgA : Gate {
 // pin/pout double-buffer the search direction: neighbouring tiles rebuild
 // p_new on their halo from p_old, so p_old must stay intact during the launch.
 template <typename T>
-void launch_cg_A2(const Geo& g, hipStream_t s, RedBuf rb, const T* src, const T* pin, T* pout, T* Ap, T* x, Scal* S,
-                  bool pointwise, int ring_slot)
+void launch_cg_A2(const Geo& g, hipStream_t s, RedBuf rb, const T* z, const T* pin, T* pout, T* Ap, T* x, Scal* S,
+                  int ring_slot)
 {
     OpCgA<T> op;
     op.gate = &S->done;
-    op.src = src;
+    op.src = z;
     op.pin = pin;
     op.pout = pout;
     op.Ap = Ap;
     op.x = x;
     op.S = S;
-    op.pointwise = pointwise;
     op.slot = ring_slot;
     run_stencil<T, 1>(g, s, op, rb);
 }
@@ -1084,50 +1400,40 @@ void launch_cg_final_x(const Geo& g, hipStream_t s, T* x, const T* p, const Scal
     run_vector<0>(g, s, op, kNoRed);
 }
 
-// r -= alpha Ap, r.r, r.(jac r)  (baseCG.hpp:154-194)
+// r -= alpha Ap, r.r  (baseCG.hpp:154-194)
 template <typename T>
 struct OpCgB : Gate {
     T* __restrict__ r;
     const T* __restrict__ Ap;
     Scal* S;
-    bool pointwise, history;
-    T alpha, jac;
+    bool history;
+    T alpha;
     struct R { T r, ap; };
-    __device__ void load()
-    {
-        alpha = (T)S->v[S_ALPHA];
-        jac = (T)S->v[S_JAC];
-    }
+    __device__ void load() { alpha = (T)S->v[S_ALPHA]; }
     template <bool NT> __device__ R fetch(long long c) const { return {ld<NT>(r + c), ld<NT>(Ap + c)}; }
     template <bool NT> __device__ void apply(long long c, const R& v, int, int, int, double* acc) const
     {
         const T rv = v.r - alpha * v.ap;
         put<NT>(r + c, rv);
         acc[0] += (double)rv * (double)rv;
-        acc[1] += (double)rv * (double)(jac * rv);
     }
     __device__ void finish(const double* t)
     {
-        if (pointwise) {
-            S->v[S_BETA] = t[1] / S->v[S_RZ];
-            S->v[S_RZ] = t[1];
-        }
         S->v[S_RR] = t[0];
         finish_iteration(S, sqrt(t[0]), history);
     }
 };
 
 template <typename T>
-void launch_cg_B(const Geo& g, hipStream_t s, RedBuf rb, T* r, const T* Ap, Scal* S, bool pointwise, bool history)
+void launch_cg_B(const Geo& g, hipStream_t s, RedBuf rb, T* r, const T* Ap, Scal* S, bool history)
 {
     OpCgB<T> op;
     op.gate = &S->done;
     op.r = r;
     op.Ap = Ap;
     op.S = S;
-    op.pointwise = pointwise;
     op.history = history;
-    run_vector<2>(g, s, op, rb);
+    run_vector<1>(g, s, op, rb);
 }
 
 template <typename T>
@@ -2096,14 +2402,9 @@ struct OpIrInit : Gate {
     float* __restrict__ x;
     float* __restrict__ p;
     Scal* SI;
-    bool pointwise;
-    float inv, jac;
+    float inv;
     struct R { float r; };
-    __device__ void load()
-    {
-        inv = (float)(1.0 / SI->v[S_INNER_NORM]);
-        jac = (float)SI->v[S_JAC];
-    }
+    __device__ void load() { inv = (float)(1.0 / SI->v[S_INNER_NORM]); }
     template <bool NT> __device__ R fetch(long long c) const { return {ld<NT>(r + c)}; }
     template <bool NT> __device__ void apply(long long c, const R& v, int, int, int, double* acc) const
     {
@@ -2112,14 +2413,12 @@ struct OpIrInit : Gate {
         put<NT>(x + c, 0.0f);
         put<NT>(p + c, 0.0f);
         acc[0] += (double)rv * (double)rv;
-        acc[1] += (double)rv * (double)(jac * rv);
     }
     __device__ void finish(const double* t)
     {
         const double e = sqrt(t[0]);
         SI->v[S_ERR0] = e;
         SI->v[S_ERR] = e;
-        SI->v[S_RZ] = t[1];
         SI->v[S_RR] = t[0];
         SI->v[S_BETA] = 0.0;
         SI->v[S_PAP_OLD] = 1.0;
@@ -2127,12 +2426,14 @@ struct OpIrInit : Gate {
         SI->v[S_AUX2] = 1e300;
         SI->fallback = 0;
         SI->restart = 0;
+        SI->passes = 0;
+        SI->recheck = 0;
         SI->iter = 0;
         SI->done = e < SI->v[S_TOL] ? 2 : 0;
     }
 };
 
-void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, float* x, float* p, Scal* SI, bool pointwise)
+void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, float* x, float* p, Scal* SI)
 {
     OpIrInit op;
     op.gate = nullptr;
@@ -2140,8 +2441,7 @@ void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, floa
     op.x = x;
     op.p = p;
     op.SI = SI;
-    op.pointwise = pointwise;
-    run_vector<2>(g, s, op, rb);
+    run_vector<1>(g, s, op, rb);
 }
 
 // ------------------------------------------------------ instantiations
@@ -2153,10 +2453,11 @@ void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, floa
     template void launch_scale_box<T>(const Geo&, hipStream_t, T*, const Scal*, int);                          \
     template void launch_fill<T>(const Geo&, hipStream_t, T*, T);                                              \
     template void launch_ghost<T>(hipStream_t, const Layout&, const Faces&, T*, int, const Scal*, const int*);  \
-    template void launch_cg_A2<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, T*, T*, T*, Scal*, bool,  \
-                                  int);                                                                            \
+    template void launch_cg_pass<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, T*, T*, T*, Scal*, bool, \
+                                    int);                                                                          \
+    template void launch_cg_A2<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, T*, T*, T*, Scal*, int);    \
     template void launch_cg_final_x<T>(const Geo&, hipStream_t, T*, const T*, const Scal*);                      \
-    template void launch_cg_B<T>(const Geo&, hipStream_t, RedBuf, T*, const T*, Scal*, bool, bool);            \
+    template void launch_cg_B<T>(const Geo&, hipStream_t, RedBuf, T*, const T*, Scal*, bool);                  \
     template void launch_cg_rz<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, Scal*);                 \
     template void launch_pointwise<T>(const Geo&, hipStream_t, const T*, T*, double, const int*);              \
     template void launch_bicg_k1<T>(const Geo&, hipStream_t, RedBuf, const T*, double, T*, const T*, Scal*);   \

@@ -74,6 +74,8 @@ struct alignas(256) Scal {
     int fallback;    // FCG: 1 once the plain preconditioner replaced the learned one
     int restart;     // FCG: 1 = discard this iteration's direction (non-finite step) and restart
     int stall_window;  // FCG: iterations per stall check (0 = off)
+    int passes;      // CG in one pass: passes that ran (iterations plus recomputed residuals)
+    int recheck;     // CG in one pass: 1 = the next pass recomputes ||r|| instead of iterating
 };
 
 // Deterministic grid reduction workspace: every block of a reducing launch
@@ -133,11 +135,11 @@ void launch_copy_flat(hipStream_t s, const double* x, double* y, long long n);
 template <typename T>
 void launch_dot(const Geo& g, hipStream_t s, RedBuf rb, const T* a, const T* b, double* out, const int* gate);
 
-// r = b - A x; S[S_ERR0 or S_ERR_OP] = ||r||, S_RZ = r.(jac r); mode 0: start of solve
+// r = b - A x; S[S_ERR0 or S_ERR_OP] = ||r||; mode 0: start of solve
 // (history[0], iteration reset, early-exit flag), mode 1: final true residual;
-// modes 2-4: residual replacement after a recursive stop (S_RR, S_ALPHA = 0, done
-// = 0 unless below tolerance or at the iteration cap), 3 also sets S_RZ (CG with a
-// pointwise preconditioner), 4 S_RHO0 = ||r||^2 (BiCGSTAB restarted with r0 = r)
+// modes 2, 3: residual replacement after a recursive stop (S_RR, S_ALPHA = 0, done
+// = 0 unless below tolerance or at the iteration cap), 3 also sets
+// S_RHO0 = ||r||^2 (BiCGSTAB restarted with r0 = r)
 void launch_residual(const Geo& g, hipStream_t s, RedBuf rb, const double* x, const double* b, double* r, Scal* S, int mode);
 
 // r = b - A x on g's region and ||r|| into *out (device); the partials go to
@@ -165,17 +167,29 @@ template <typename T>
 void launch_ghost(hipStream_t s, const Layout& L, const Faces& F, T* field, int with_flux, const Scal* S,
                   const int* gate);
 
-// ---- CG (plain / pointwise-preconditioned / buffer-preconditioned) ----
-// p_new = a*src + beta*p_old (a = S_JAC or 1), Ap = A p_new, pAp -> alpha = S_RZ / pAp,
+// ---- CG with a pointwise preconditioner: one pass per iteration ----
+// One launch is one iteration (see k_cg_pass): r_out = r_in - alpha_prev A pin,
+// pout = jac r_out + beta pin, A pout and the iteration's sums, whose finish
+// sets alpha, beta, the residual norm and the convergence flag.  r_in/r_out
+// and pin/pout must be distinct buffers holding 0 off the solver region.
+// ring_slot >= 0: alpha goes to S->ahist[ring_slot] for launch_fcg_flush and x
+// is not touched; otherwise x += alpha_prev pin (the caller adds the last step).
+// The buffers alternate with S->passes: pass n (from 0) reads what pass n - 1 wrote.
+template <typename T>
+void launch_cg_pass(const Geo& g, hipStream_t s, RedBuf rb, const T* r_in, const T* pin, T* r_out, T* pout, T* x,
+                    Scal* S, bool history, int ring_slot);
+
+// ---- CG with a buffer preconditioner ----
+// p_new = z + beta*p_old, Ap = A p_new, pAp -> alpha = S_RZ / pAp,
 // and the previous iteration's solution update x += alpha_prev p_old on the
 // tile's own points.  pin/pout must be distinct buffers (halo tiles rebuild
 // p_new from p_old).
 template <typename T>
-void launch_cg_A2(const Geo& g, hipStream_t s, RedBuf rb, const T* src, const T* pin, T* pout, T* Ap, T* x, Scal* S,
-                  bool pointwise, int ring_slot = -1);  // ring_slot >= 0: as launch_fcg_p_fused's
-// r -= alpha Ap, rr (and r.(jac r) when pointwise) -> err, beta, iter, done
+void launch_cg_A2(const Geo& g, hipStream_t s, RedBuf rb, const T* z, const T* pin, T* pout, T* Ap, T* x, Scal* S,
+                  int ring_slot = -1);  // ring_slot >= 0: as launch_fcg_p_fused's
+// r -= alpha Ap, rr -> err, iter, done
 template <typename T>
-void launch_cg_B(const Geo& g, hipStream_t s, RedBuf rb, T* r, const T* Ap, Scal* S, bool pointwise, bool history);
+void launch_cg_B(const Geo& g, hipStream_t s, RedBuf rb, T* r, const T* Ap, Scal* S, bool history);
 // x += S[S_ALPHA] p: the last iteration's solution update, after the loop
 template <typename T>
 void launch_cg_final_x(const Geo& g, hipStream_t s, T* x, const T* p, const Scal* S);
@@ -272,8 +286,8 @@ void launch_ir_residual(const Geo& g, hipStream_t s, RedBuf rb, const double* x,
                         Scal* SI, double itol, double itol0, double adapt);
 // x += ||r32|| * d on the solver region (the inner solve's un-normalisation)
 void launch_ir_update(const Geo& g, hipStream_t s, double* x, const float* d, const Scal* SI);
-// inner start: r = r32 / ||r32||, x = 0, p = 0, err0, rz (pointwise jac) -> SI
-void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, float* x, float* p, Scal* SI, bool pointwise);
+// inner start: r = r32 / ||r32||, x = 0, p = 0, err0 -> SI
+void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, float* x, float* p, Scal* SI);
 
 }  // namespace pps
 
