@@ -191,10 +191,10 @@ int pps_rhs_spectrum(void* ctx, uint64_t seed, int kmax, int accumulate);
 /* ---- measurement ------------------------------------------------------- */
 /* kernel ids for pps_time_kernel */
 enum {
-    PPS_K_CG_STENCIL = 0,   /* fused p = z + beta p, Ap = A p, p.Ap (x's updates deferred to a
-                               pass per 16 iterations, as CG runs it where the device holds
-                               the directions' ring) */
-    PPS_K_CG_UPDATE = 1,    /* r -= alpha Ap, r.r, r.z                    */
+    PPS_K_CG_STENCIL = 0,   /* fused p = z + beta p, Ap = A p, p.Ap, of CG with a buffer
+                               preconditioner (x's updates deferred to a pass per 16
+                               iterations, as it runs where the device holds the directions' ring) */
+    PPS_K_CG_UPDATE = 1,    /* r -= alpha Ap, r.r, of the same            */
     PPS_K_RESIDUAL = 2,     /* r = b - A x, r.r                           */
     PPS_K_COPY = 3,         /* plain copy of the solver region (reference) */
     PPS_K_CHEB_SWEEP = 4,   /* Chebyshev sweep                            */
@@ -218,11 +218,11 @@ int pps_time_kernel(void* ctx, int kernel, int reps, double* ms, double* bytes);
  * automatic (non-temporal once a field exceeds 32 MiB), 1 always
  * non-temporal, -1 never. */
 int pps_set_tiling(void* ctx, int kz_stencil, int nontemporal);
-/* Chebyshev sweeps: pairs = 1 runs them two per pass (one fused kernel reads
- * y_c, y_{c-1} and B once and writes y_{c+1} and y_{c+2}; the default), 0 one
- * sweep per pass; kz = z-chunk of the fused kernel (0 keeps the current one,
- * -1 returns to the automatic choice: the longest of 64/32/16 planes giving
- * 1024 blocks).
+/* Chebyshev sweeps: pairs = 1 runs the recurrence's start and its sweeps two or
+ * three per pass (one fused kernel reads y_c, y_{c-1} and B once and writes the
+ * last two of them; the default), 0 one sweep per pass; kz = z-chunk of the
+ * fused kernel (0 keeps the current one, -1 returns to the automatic choice,
+ * the chunk that leaves the busiest compute unit the least work).
  * No counterpart in the reference: its sweeps are one kernel each
  * (kernelsAlpakaChebyshev.hpp:191-273). */
 int pps_set_cheb_pairs(void* ctx, int pairs, int kz);

@@ -344,7 +344,8 @@ class Context:
         self._chk(lib().pps_set_deferred_x(self.h, int(bool(on))))
 
     def set_cheb_pairs(self, pairs=1, kz=0):
-        """Chebyshev sweeps two per pass (1, the default) or one per pass (0); kz: z-chunk of the fused kernel."""
+        """Chebyshev sweeps two or three per pass (1, the default) or one per pass (0); kz: z-chunk of the fused
+        kernel."""
         self._chk(lib().pps_set_cheb_pairs(self.h, int(pairs), int(kz)))
 
     def set_tiling(self, kz_stencil=0, nontemporal=0):

@@ -117,9 +117,9 @@ struct Ctx {
     int nt = 0;       // non-temporal stores of field outputs
     int nt_mode = 0;  // 0: automatic (nt_auto), 1: always, -1: never
     int nt_auto = 0;  // the fields' working set exceeds the last-level cache
-    int cheb_pairs = 1;  // Chebyshev sweeps run two per pass (k_cheb_pair)
+    int cheb_pairs = 1;  // Chebyshev sweeps run two or three per pass (k_cheb_multi)
     int deferred_x = 1;  // Krylov stages keep a ring of directions where the device holds it
-    int cheb_kz = 0;     // z-chunk of the fused Chebyshev pair (0: chosen per launch)
+    int cheb_kz = 0;     // z-chunk of the fused Chebyshev sweeps (0: chosen per launch)
     double* stage_d = nullptr;  // dense planes on their way between pageable host memory and a pitched field
     int stage_planes = 0;
     std::string err;
@@ -159,8 +159,9 @@ struct Ctx {
         cg.kz = cheb_kz;
         return cg;
     }
-    // the fused pair needs the Neumann mirror point (two cells inward) inside the data region
-    bool cheb_pairs_ok() const { return cheb_pairs && np[0] >= 2 && np[1] >= 2 && np[2] >= 2; }
+    // the kernels that address a tile's rows (at most 40) with 31-bit byte offsets
+    bool tile_offsets_ok() const { return 40ll * 8 * L64.px < 0x7fffffffll; }
+    bool cheb_fused_ok() const { return cheb_pairs && tile_offsets_ok(); }
 
     int alloc_field(Field& f, int prec)
     {
@@ -409,7 +410,7 @@ struct JacobiStage : Stage {
 
 struct ChebStage : Stage {
     double theta = 0, delta = 0, sigma = 0;
-    Field Y, Z, W, V, Bc;  // V: fourth iterate buffer of fused pairs; Bc: FP32 copy of the input
+    Field Y, Z, W, V, Bc;  // V: fourth iterate buffer of the fused sweeps; Bc: FP32 copy of the input
     ChebStage(Ctx& c, const pps_stage& s, int l) : Stage(c, s, l)
     {
         // chebyshevIteration.hpp:22-26 (global, rescaled); alpaka local form
@@ -430,7 +431,7 @@ struct ChebStage : Stage {
         int rc = C.get_work(k + ".Y", P, Y);
         if (!rc) rc = C.get_work(k + ".Z", P, Z);
         if (!rc) rc = C.get_work(k + ".W", P, W);
-        if (!rc && C.cheb_pairs_ok()) rc = C.get_work(k + ".V", P, V);
+        if (!rc && C.cheb_fused_ok()) rc = C.get_work(k + ".V", P, V);
         if (!rc && P == 32) rc = C.get_work(k + ".B", 32, Bc);
         return rc;
     }
@@ -441,8 +442,6 @@ struct ChebStage : Stage {
         // three-term recurrence; the reference returns -W after its final
         // rotation, which is -y_{m-1} (chebyshevIteration.hpp:93-128): the two
         // sweeps computing y_m and y_{m+1} do not reach the output and are skipped.
-        // Sweeps c = 2 .. m-2 run two per pass (k_cheb_pair) where the grid
-        // allows it, one first when their number is odd.
         const int m = cfg.max_iter;
         const Geo g = C.gsolver(sizeof(T) == 4 ? 32 : 64);
         double rhoOld = 1 / sigma;
@@ -460,12 +459,7 @@ struct ChebStage : Stage {
         T* Zp = static_cast<T*>(Zf.p);
         T* Wp = static_cast<T*>(Wf.p);
         T* Vp = static_cast<T*>(Vf.p);
-        const bool pairs = C.cheb_pairs_ok() && Vp != nullptr;
-        const ChebPairGeo cg = C.cheb_pair_geo();
-        launch_cheb_first<T>(g, C.stream, B, Zp, Yp, c0, c1, gate);
-        Field yf;
-        yf.prec = sizeof(T) == 4 ? 32 : 64;
-        double a[2], b[2], cz[2];
+        double a[3], b[3], cz[3];
         auto next = [&](int q) {
             rhoOld = rhoCurr;
             rhoCurr = 1 / (2 * sigma - rhoOld);
@@ -473,37 +467,44 @@ struct ChebStage : Stage {
             b[q] = rhoCurr * 2 / delta;
             cz[q] = rhoCurr * rhoOld;
         };
-        for (int c = 2; c <= m - 2;) {
-            const int left = m - 2 - c + 1;
+        if (C.cheb_fused_ok() && Vp != nullptr) {
+            // m - 2 levels, the start and the sweeps c = 2 .. m-2, three per
+            // pass; a remainder of 1 or 2 is taken in passes of two
+            const ChebPairGeo cg = C.cheb_pair_geo();
+            bool start = true;
+            for (int left = m - 2; left > 0;) {
+                const int n = left % 3 == 0 ? 3 : 2;
+                for (int l = 0; l < n; ++l)
+                    if (!(start && l == 0)) next(l);
+                const T* Yin = start ? B : Yp;
+                const T* Zin = start ? nullptr : Zp;
+                left -= n;
+                if (left == 0) {
+                    launch_cheb_multi<T, TO>(g, cg, C.stream, n, Yin, Zin, B, nullptr, X, a, b, cz, c0, c1, -1.0, gate);
+                } else {
+                    launch_cheb_multi<T, T>(g, cg, C.stream, n, Yin, Zin, B, Wp, Vp, a, b, cz, c0, c1, 1.0, gate);
+                    std::swap(Yp, Vp);  // the last level is the next pass's Y, the one before its Z
+                    std::swap(Zp, Wp);
+                }
+                start = false;
+            }
+            return;
+        }
+        launch_cheb_first<T>(g, C.stream, B, Zp, Yp, c0, c1, gate);
+        Field yf;
+        yf.prec = sizeof(T) == 4 ? 32 : 64;
+        for (int c = 2; c <= m - 2; ++c) {
             yf.p = Yp;
             C.ghost(yf, false, nullptr, gate);
-            if (pairs && left % 2 == 0) {
-                next(0);
-                next(1);
-                if (left > 2) {
-                    launch_cheb_pair<T, T>(g, cg, C.stream, Yp, Zp, B, Wp, Vp, a, b, cz, 1.0, false, gate);
-                    T* y = Yp;  // y_{c+2} -> Y, y_{c+1} -> Z
-                    T* z = Zp;
-                    Yp = Vp;
-                    Zp = Wp;
-                    Wp = y;
-                    Vp = z;
-                } else {
-                    launch_cheb_pair<T, TO>(g, cg, C.stream, Yp, Zp, B, Wp, X, a, b, cz, -1.0, true, gate);
-                }
-                c += 2;
+            next(0);
+            if (c < m - 2) {
+                launch_cheb_sweep<T, T>(g, C.stream, Yp, B, Zp, Wp, a[0], b[0], cz[0], 1.0, gate);
+                T* t = Zp;  // swap(Z,Y); swap(W,Y)
+                Zp = Yp;
+                Yp = Wp;
+                Wp = t;
             } else {
-                next(0);
-                if (c < m - 2) {
-                    launch_cheb_sweep<T, T>(g, C.stream, Yp, B, Zp, Wp, a[0], b[0], cz[0], 1.0, gate);
-                    T* t = Zp;  // swap(Z,Y); swap(W,Y)
-                    Zp = Yp;
-                    Yp = Wp;
-                    Wp = t;
-                } else {
-                    launch_cheb_sweep<T, TO>(g, C.stream, Yp, B, Zp, X, a[0], b[0], cz[0], -1.0, gate);
-                }
-                c += 1;
+                launch_cheb_sweep<T, TO>(g, C.stream, Yp, B, Zp, X, a[0], b[0], cz[0], -1.0, gate);
             }
         }
     }
@@ -2077,9 +2078,9 @@ int pps_time_kernel(void* ctx, int kernel, int reps, double* ms, double* bytes)
         case PPS_K_COPY_FLAT: launch_copy_flat(C->stream, a.d(), e.d(), C->L64.total); break;
         case PPS_K_CHEB_PAIR: {
             const double ca[2] = {0.1, 0.15}, cb[2] = {0.2, 0.25}, cc[2] = {0.3, 0.35};
-            launch_cheb_pair<double, double>(g, C->cheb_pair_geo(), C->stream, (it & 1) ? d.d() : a.d(), b.d(), c.d(),
-                                             (it & 1) ? e.d() : d.d(), (it & 1) ? a.d() : e.d(), ca, cb, cc, 1.0, false,
-                                             nullptr);
+            launch_cheb_multi<double, double>(g, C->cheb_pair_geo(), C->stream, 2, (it & 1) ? d.d() : a.d(), b.d(), c.d(),
+                                              (it & 1) ? e.d() : d.d(), (it & 1) ? a.d() : e.d(), ca, cb, cc, 1.0, 1.0,
+                                              1.0, nullptr);
             break;
         }
         }

@@ -19,7 +19,8 @@
 //    for FP64 operands, 128 threads x 4 points for FP32) for the fused
 //    axpy/dot updates: all of a thread's loads are issued before its store,
 //    and consecutive blocks stream consecutive addresses.
-// A third, k_cheb_pair, runs two Chebyshev sweeps per pass.
+// k_cg_pass runs one CG iteration and k_cheb_multi two or three Chebyshev
+// sweeps per pass.
 //
 // Reductions are FP64 in every precision and deterministic: DPP row
 // butterflies inside each wavefront, LDS across the wavefronts, one partial
@@ -993,6 +994,79 @@ void launch_ghost(hipStream_t s, const Layout& L, const Faces& F, T* field, int 
     hipLaunchKernelGGL(k_ghost<T>, grid, dim3(256), 0, s, L, F, field, with_flux, S, gate);
 }
 
+// ------------------------------------ pieces of the multi-level marching kernels
+// (k_cg_pass, k_cheb_multi: several applications of A per pass, on a tile and rings around it)
+
+template <typename T>
+__device__ __forceinline__ T lap7(T v, T xm, T xp, T ym, T yp, T zm, T zp, T cx, T cy, T cz)
+{
+    const T dx = (xm - v) + (xp - v), dy = (ym - v) + (yp - v), dz = (zm - v) + (zp - v);
+    return fma(cx, dx, fma(cy, dy, cz * dz));
+}
+
+// Raw buffer access to one plane of a field, relative to a tile's origin: a load
+// whose byte offset is at or beyond num_records returns 0 and such a store is
+// dropped, so points off the solver region (offset kOob) and planes off it
+// (num_records 0) need no branch and no mask around the access.  The aux bit
+// stores non-temporally.
+constexpr unsigned kOob = 0x80000000u;
+constexpr int kInRange = 0x7fffffff;
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const T* p, bool ok)
+{
+    const unsigned long long a = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+    void* q = (void*)(((unsigned long long)hi << 32) | lo);
+    return __builtin_amdgcn_make_buffer_rsrc(q, (short)0, ok ? kInRange : 0, 0x00020000);
+}
+template <typename T>
+__device__ __forceinline__ T buf_ld(__amdgpu_buffer_rsrc_t r, unsigned off)
+{
+    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t r, unsigned off, T v)
+{
+    if constexpr (sizeof(T) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, v), r, off, 0, NT ? 2 : 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, 0, NT ? 2 : 0);
+}
+
+// point t of the ring around a box of W x H points -> (row, col) in the box's frame
+template <int W, int H>
+__device__ __forceinline__ void ring_point(int t, int& r, int& c)
+{
+    if (t < W + 2) { r = -1; c = t - 1; }
+    else if (t < 2 * (W + 2)) { r = H; c = t - (W + 2) - 1; }
+    else if (t < 2 * (W + 2) + H) { r = t - 2 * (W + 2); c = -1; }
+    else { r = t - 2 * (W + 2) - H; c = W; }
+}
+
+// z-chunk of a marching kernel whose blocks load `extra` planes beyond their
+// own and of which `slots` run at once: the one with the least work in the
+// busiest slot, ceil(blocks / slots) * (kz + extra) planes (the longest of
+// equals, up to 128 planes)
+static int pick_kz(long long tiles, int nz, int slots, int extra)
+{
+    int best = 1;
+    long long cost = -1;
+    for (int kz = 1; kz <= 128; ++kz) {
+        if (kz > 1 && kz > nz) break;
+        const long long nb = tiles * ((nz + kz - 1) / kz);
+        const long long c = ((nb + slots - 1) / slots) * (std::min(kz, nz) + extra);
+        if (cost < 0 || c <= cost) {
+            cost = c;
+            best = kz;
+        }
+    }
+    return best;
+}
+
+constexpr int kCUs = 256;  // compute units of the MI355X
+
 // ------------------------------------------------------------------- CG
 
 // One CG iteration in one pass over the grid (pointwise preconditioner M = jac I;
@@ -1029,13 +1103,6 @@ void launch_ghost(hipStream_t s, const Layout& L, const Faces& F, T* field, int 
 constexpr double kCgRecheck = 1e-2;  // beta's relative error stays near eps / kCgRecheck
 constexpr int kCgW = 8;              // wavefronts per block
 
-template <typename T>
-__device__ __forceinline__ T lap7(T v, T xm, T xp, T ym, T yp, T zm, T zp, T cx, T cy, T cz)
-{
-    const T dx = (xm - v) + (xp - v), dy = (ym - v) + (yp - v), dz = (zm - v) + (zp - v);
-    return fma(cx, dx, fma(cy, dy, cz * dz));
-}
-
 // p = z + beta p_old with z = jac r, each product rounded, as the reference
 // forms it (baseCG.hpp:139,199-203)
 template <typename T>
@@ -1055,16 +1122,6 @@ struct CgPassArgs {
     T* __restrict__ x;  // null: x's updates are deferred to the ring's flush
     const Scal* S;
 };
-
-// point t of the ring around a box of W x H points -> (row, col) in the box's frame
-template <int W, int H>
-__device__ __forceinline__ void ring_point(int t, int& r, int& c)
-{
-    if (t < W + 2) { r = -1; c = t - 1; }
-    else if (t < 2 * (W + 2)) { r = H; c = t - (W + 2) - 1; }
-    else if (t < 2 * (W + 2) + H) { r = t - 2 * (W + 2); c = -1; }
-    else { r = t - 2 * (W + 2) - H; c = W; }
-}
 
 template <typename T, int RY, bool XUPD, bool NT>
 __global__ __launch_bounds__(kTX* kCgW) void k_cg_pass(Geo g, CgPassArgs<T> A, RedBuf rb)
@@ -1264,28 +1321,6 @@ struct OpCgPass {
     }
 };
 
-// z-chunk of a marching kernel whose blocks load `extra` planes beyond their
-// own and of which `slots` run at once: the one with the least work in the
-// busiest slot, ceil(blocks / slots) * (kz + extra) planes (the longest of
-// equals, up to 128 planes)
-static int pick_kz(long long tiles, int nz, int slots, int extra)
-{
-    int best = 1;
-    long long cost = -1;
-    for (int kz = 1; kz <= 128; ++kz) {
-        if (kz > 1 && kz > nz) break;
-        const long long nb = tiles * ((nz + kz - 1) / kz);
-        const long long c = ((nb + slots - 1) / slots) * (std::min(kz, nz) + extra);
-        if (cost < 0 || c <= cost) {
-            cost = c;
-            best = kz;
-        }
-    }
-    return best;
-}
-
-constexpr int kCUs = 256;  // compute units of the MI355X
-
 template <typename T, int RY>
 static void run_cg_pass(const Geo& g, hipStream_t s, const CgPassArgs<T>& A, const OpCgPass& op, RedBuf rb)
 {
@@ -1314,7 +1349,9 @@ void launch_cg_pass(const Geo& g0, hipStream_t s, RedBuf rb, const T* r_in, cons
     // where there is enough work for two 16-plane chunks per CU, 16-row tiles (two
     // blocks per CU) below that.  us per iteration, 32 / 16 rows, FP64: 514^3
     // 1110 / 1169, 258^3 145 / 148, 194^3 77.5 / 71.5, 130^3 32.8 / 27.1, 66^3 15.5 / 13.9
-    if (tiles(4 * kCgW) * nz >= 2ll * 16 * kCUs) run_cg_pass<T, 4>(tiling(4 * kCgW, kCUs), s, A, op, rb);
+    // (and where the last row of 32-row tiles is more than half full)
+    const bool tall = tiles(4 * kCgW) * nz >= 2ll * 16 * kCUs && (ny - 1) % (4 * kCgW) + 1 > 2 * kCgW;
+    if (tall) run_cg_pass<T, 4>(tiling(4 * kCgW, kCUs), s, A, op, rb);
     else run_cg_pass<T, 2>(tiling(2 * kCgW, 2 * kCUs), s, A, op, rb);
 }
 
@@ -1648,6 +1685,19 @@ void launch_bicg_k6(const Geo& g, hipStream_t s, T* p, const T* r, const T* AMp,
 
 // ------------------------------------------------------------ Chebyshev
 
+// one level: a v + b (B + A v) - c z
+template <typename T>
+__device__ __forceinline__ T cheb_level(T a, T v, T b, T rhs, T Av, T c, T z)
+{
+    return fma(-c, z, fma(b, rhs + Av, a * v));
+}
+// the recurrence's start: c1 (2 B + c0 A B)
+template <typename T>
+__device__ __forceinline__ T cheb_start(T c1, T c0, T v, T Av)
+{
+    return c1 * fma(c0, Av, T(2) * v);
+}
+
 // Z = c0 B ; Y = c1 (2B + c0 A B)   (chebyshevIteration.hpp:79-90)
 template <typename T>
 struct OpChebFirst : Gate {
@@ -1660,7 +1710,7 @@ struct OpChebFirst : Gate {
     template <bool NT> __device__ void out(long long c, T vc, T Av, double*) const
     {
         put<NT>(Z + c, c0 * vc);
-        put<NT>(Y + c, c1 * (T(2) * vc + c0 * Av));
+        put<NT>(Y + c, cheb_start(c1, c0, vc, Av));
     }
     __device__ void finish(const double*) {}
 };
@@ -1689,7 +1739,7 @@ struct OpChebFirstOut : Gate {
     __device__ T in(long long c) const { return B[c]; }
     template <bool NT> __device__ void out(long long c, T vc, T Av, double*) const
     {
-        const T y = which == 0 ? c0 * vc : c1 * (T(2) * vc + c0 * Av);
+        const T y = which == 0 ? c0 * vc : cheb_start(c1, c0, vc, Av);
         put<NT>(X + c, (TO)(sign * (double)y));
     }
     __device__ void finish(const double*) {}
@@ -1725,7 +1775,7 @@ struct OpChebSweep : Gate {
     template <bool NT> __device__ Ox out_raw(long long c) const { return {ld<NT>(B + c), ld<NT>(Z + c)}; }
     template <bool NT> __device__ void out(long long c, T vc, T Av, const T&, const Ox& o, double*) const
     {
-        const T w = a * vc + b * (o.b + Av) - cz * o.z;
+        const T w = cheb_level(a, vc, b, o.b, Av, cz, o.z);
         if constexpr (sizeof(TO) == sizeof(T)) put<NT>(W + c, sign < 0 ? -w : w);
         else put<NT>(W + c, (TO)(sign * (double)w));
     }
@@ -1749,261 +1799,402 @@ void launch_cheb_sweep(const Geo& g, hipStream_t s, const T* Y, const T* B, cons
     run_stencil<T, 0>(g, s, op, kNoRed);
 }
 
-// ---------------------------------------------- fused pair of Chebyshev sweeps
-// Two consecutive sweeps of the three-term recurrence in one pass over the grid
-// (temporal blocking of chebyshevIteration.hpp:103-113 / the alpaka
+// ---------------------------------------------- fused Chebyshev sweeps
+// S = 2 or 3 consecutive sweeps of the three-term recurrence in one pass over
+// the grid (temporal blocking of chebyshevIteration.hpp:103-113 / the alpaka
 // Chebyshev2Kernel, kernelsAlpakaChebyshev.hpp:191-273):
-//   W1 = a1 Y  + b1 (B + A Y)  - c1 Z      sweep c    (Y = y_c, Z = y_{c-1})
-//   W2 = a2 W1 + b2 (B + A W1) - c2 Y      sweep c+1
-// with the Neumann ghosts of W1 reset between the two as the unfused sweeps
-// reset those of their input (ghost = the data point two cells inward).  A
-// block owns a 64 x 32 tile of W2 and marches z; it computes W1 on the tile
-// plus a one-point ring (the neighbours W2 needs), from Y on the tile plus a
-// two-point ring.  Per plane: the Y plane is staged in LDS (x-y neighbours),
-// each point's z history lives in the registers of the thread that owns it
-// (tile points: 4 rows per thread; ring points: one per thread), W1 of plane
-// s goes to LDS and W2 of plane s-1 comes out of it.  HBM traffic per pair:
-// Y, Z, B read once (plus the rings and the two halo planes), W1 and W2
-// written once: 5 fields in place of the 8 of two separate sweeps.
-#ifndef PPS_CHEB_WAVES
-#define PPS_CHEB_WAVES 8
-#endif
-constexpr int kCpW = PPS_CHEB_WAVES;       // wavefronts per block (tile rows ly + kCpW q)
-constexpr int kCpT = kTX * kCpW;           // threads per block
-constexpr int kCpRY = 4;                   // tile rows per thread
-constexpr int kCpTY = kCpW * kCpRY;        // tile height
-constexpr int kCpE1X = kTX + 2, kCpE1Y = kCpTY + 2;  // W1 region: tile + 1
-constexpr int kCpE2X = kTX + 4, kCpE2Y = kCpTY + 4;  // Y region: tile + 2
-constexpr int kCpRing1 = 2 * kCpE1X + 2 * kCpTY;      // W1 ring points (164)
-constexpr int kCpRing2 = 2 * kCpE2X + 2 * kCpE1Y;     // outer Y ring points (172)
-static_assert(kCpRing1 <= kCpT && kCpRing2 <= kCpT, "ring points need one thread each");
+//   W1 = a1 Y  + b1 (B + A Y)  - c1 Z      sweep c      (Y = y_c, Z = y_{c-1})
+//   W2 = a2 W1 + b2 (B + A W1) - c2 Y      sweep c + 1
+//   W3 = a3 W2 + b3 (B + A W2) - c3 W1     sweep c + 2
+// The stage's first pass reads only B: Z = c0 B, Y-stream B, and its first level
+// is the recurrence's start W1 = c1 (2 B + c0 A B).  A pass reads Y, Z, B and
+// writes the last two levels (the stage's last pass only its result): 5 words
+// per point for 2 or 3 sweeps, where separate sweeps move 4 each.
+//
+// A block owns a 64 x (8 RY) tile and marches z.  Level l is formed on the tile
+// and S - l rings of points around it, at plane s - (l - 1) of step s; a thread
+// owns RY consecutive rows of one column (their y-neighbours are its own
+// registers) and at most one point of each ring, with each point's z-history in
+// registers.  The x-y neighbours of every level go through LDS, two planes per
+// level used in turn, with one barrier per plane: level l of a plane is read
+// one step after it was written, and its buffer is rewritten a step later.
+//
+// Neumann ghosts (the data point two cells inward) are never stored: the thread
+// that owns a ghost position loads and evaluates its mirror point instead and
+// puts the value at the ghost's place in LDS; ghosts in z are a choice of
+// register.  A level's other points off the solver region are 0; B's, which the
+// first pass's start reads, are whatever the field holds there.
+//
+// Measured at 512^3 FP64: three sweeps in 1.30 ms (4.1 TB/s of its 5 words; 4.5
+// with the rings' re-reads that miss L2), 0.43 ms per sweep, where the pair took
+// 1.08 ms and needed a ghost fill per pass with Neumann faces.  The instruction
+// issue is a third of the time; the waves wait for memory and the barrier.
+constexpr int kChW = 8;   // wavefronts per block
 
-// ring1 point t -> (row, col) of the W1 region; ring2 point t -> (row, col) of the Y region
-__device__ __forceinline__ void cp_ring1(int t, int& r, int& c)
-{
-    if (t < kCpE1X) { r = 0; c = t; }
-    else if (t < 2 * kCpE1X) { r = kCpE1Y - 1; c = t - kCpE1X; }
-    else if (t < 2 * kCpE1X + kCpTY) { r = 1 + t - 2 * kCpE1X; c = 0; }
-    else { r = 1 + t - 2 * kCpE1X - kCpTY; c = kCpE1X - 1; }
-}
-__device__ __forceinline__ void cp_ring2(int t, int& r, int& c)
-{
-    if (t < kCpE2X) { r = 0; c = t; }
-    else if (t < 2 * kCpE2X) { r = kCpE2Y - 1; c = t - kCpE2X; }
-    else if (t < 2 * kCpE2X + kCpE1Y) { r = 1 + t - 2 * kCpE2X; c = 0; }
-    else { r = 1 + t - 2 * kCpE2X - kCpE1Y; c = kCpE2X - 1; }
-}
+template <typename T, typename TO>
+struct ChebArgs {
+    const T* __restrict__ Y;   // first pass: B
+    const T* __restrict__ Z;   // null: first pass
+    const T* __restrict__ B;
+    T* __restrict__ Wp;        // level S - 1 (null: the stage's last pass)
+    TO* __restrict__ W;        // level S
+    T a[3], b[3], c[3], c0, c1;
+    T sign;                    // of W
+    const int* gate;
+};
 
-template <typename T, typename TO, bool NT, bool LAST>
-__global__ __launch_bounds__(kCpT) void k_cheb_pair(Geo g, ChebPairGeo cg, const T* __restrict__ Y,
-                                                        const T* __restrict__ Z, const T* __restrict__ B,
-                                                        T* __restrict__ W1, TO* __restrict__ W2, T a1, T b1, T c1,
-                                                        T a2, T b2, T c2, double sign, const int* gate)
+// registers of one owned point: Y of planes s-1..s+2, Z of s, s+1, B of s-2..s+1, levels 1 and 2
+template <typename T>
+struct ChebPoint {
+    T ym, yc, yp, yn, zc, zn, b2, b1, bc, bn, um, uc, un, vm, vc, vn;
+};
+
+// NEU: the grid has Neumann faces
+template <typename T, typename TO, int S, int RY, bool NEU, bool NT>
+__global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) void k_cheb_multi(Geo g, ChebPairGeo cg, ChebArgs<T, TO> A)
 {
-    if (gate != nullptr && *gate != 0) return;
-    __shared__ T ysl[2][kCpE2Y][kCpE2X];
-    __shared__ T wsl[2][kCpE1Y][kCpE1X];
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int tx0 = b % g.ntx, rr = b / g.ntx;
+    if (A.gate != nullptr && *A.gate != 0) return;
+    constexpr int TY = kChW * RY;
+    // points of ring d around the tile
+    constexpr int NR[3] = {2 * (kTX + 2) + 2 * TY, 2 * (kTX + 4) + 2 * (TY + 2), 2 * (kTX + 6) + 2 * (TY + 4)};
+    static_assert(NR[2] <= kTX * kChW, "ring points need one thread each");
+    __shared__ T ysl[2][TY + 2 * S][kTX + 2 * S];
+    __shared__ T usl[2][TY + 2 * (S - 1)][kTX + 2 * (S - 1)];                                  // level 1
+    __shared__ T vsl[S == 3 ? 2 : 1][S == 3 ? TY + 2 : 1][S == 3 ? kTX + 2 : 1];               // level 2
+    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int tx0 = bid % g.ntx, rr = bid / g.ntx;
     const int ty0 = rr % g.nty, tz0 = rr / g.nty;
-    const int i0 = g.lo0 + tx0 * kTX, j0 = g.lo1 + ty0 * kCpTY;
+    const int i0 = g.lo0 + tx0 * kTX, j0 = g.lo1 + ty0 * TY;
     const int k0 = g.lo2 + tz0 * g.kz, k1 = min(k0 + g.kz, g.hi2);
-    const int tid = threadIdx.x + kTX * threadIdx.y;
-    const int lx = threadIdx.x, ly = threadIdx.y;
-    const T cx = (T)g.cx, cy = (T)g.cy, czz = (T)g.cz;
-    auto solver = [&](int i, int j, int k) {
-        return i >= g.lo0 && i < g.hi0 && j >= g.lo1 && j < g.hi1 && k >= g.lo2 && k < g.hi2;
-    };
-    auto inbox = [&](int i, int j, int k) {
-        return i >= 0 && i < cg.ng[0] && j >= 0 && j < cg.ng[1] && k >= 0 && k < cg.ng[2];
-    };
-    auto at = [&](int i, int j, int k) { return (long long)g.ox + i + (long long)g.px * j + g.plane * k; };
-    auto yld = [&](int i, int j, int k) { return inbox(i, j, k) ? Y[at(i, j, k)] : T(0); };
+    const int lx = threadIdx.x, ly = threadIdx.y, tid = lx + kTX * ly;
+    const T cx = (T)g.cx, cy = (T)g.cy, cz = (T)g.cz;
+    const bool first = A.Z == nullptr;
 
-    // tile points: (i0 + lx, j0 + ly + kCpW q)
-    const int ic = i0 + lx;
-    T ym[kCpRY], yc[kCpRY], yp[kCpRY], yn[kCpRY], zc[kCpRY], zn[kCpRY], bc[kCpRY], bn[kCpRY], bp[kCpRY];
-    T wm[kCpRY], wc[kCpRY], wn[kCpRY];
-    // W1 ring point (one per thread t < kCpRing1) and outer Y ring point (t < kCpRing2)
-    int r1r = 0, r1c = 0, r2r = 0, r2c = 0;
-    const bool has1 = tid < kCpRing1, has2 = tid < kCpRing2;
-    if (has1) cp_ring1(tid, r1r, r1c);
-    if (has2) cp_ring2(tid, r2r, r2c);
-    const int i1 = i0 - 1 + r1c, j1 = j0 - 1 + r1r;  // ring1 point
-    const int i2 = i0 - 2 + r2c, j2 = j0 - 2 + r2r;  // ring2 point
-    T qm = 0, qc = 0, qp = 0, qn = 0, qz = 0, qzn = 0, qb = 0, qbn = 0;
-    T oc = 0, on = 0;
+    // a ghost position stands for its mirror point
+    auto mirx = [&](int i) {
+        if constexpr (!NEU) return 0;
+        return (cg.neu & 1) && i == cg.lo_d[0] - 1 ? 2 : (cg.neu & 2) && i == cg.hi_d[0] ? -2 : 0;
+    };
+    auto miry = [&](int j) {
+        if constexpr (!NEU) return 0;
+        return (cg.neu & 4) && j == cg.lo_d[1] - 1 ? 2 : (cg.neu & 8) && j == cg.hi_d[1] ? -2 : 0;
+    };
+    auto inxy = [&](int i, int j) { return i >= g.lo0 && i < g.hi0 && j >= g.lo1 && j < g.hi1; };
+    auto ybox = [&](int i, int j) { return i >= 0 && i < cg.ng[0] && j >= 0 && j < cg.ng[1]; };
+    // byte offset of tile point (r, c) from the fields' tile origin (row -S, column -S)
+    auto off = [&](int r, int c) { return (unsigned)(g.px * (r + S) + c + S) * (unsigned)sizeof(T); };
+    const long long org = (long long)g.ox + (i0 - S) + (long long)g.px * (j0 - S);
 
-    const int s0 = k0 - 1;
+    // tile rows: row q at j0 + ly RY + q; `val` = the (mirrored) point is in the
+    // solver region; `to` its offset for loads (kOob where nothing is read), `so`
+    // the point's own offset for stores (kOob off the solver region)
+    const int jr = ly * RY, dc = mirx(i0 + lx);
+    int dr[RY];
+    bool val[RY];
+    unsigned to[RY], so[RY];
 #pragma unroll
-    for (int q = 0; q < kCpRY; ++q) {
-        const int j = j0 + ly + kCpW * q;
-        ym[q] = yld(ic, j, s0 - 1);
-        yc[q] = yld(ic, j, s0);
-        yp[q] = yld(ic, j, s0 + 1);
-        const bool sv = solver(ic, j, s0);
-        zc[q] = sv ? Z[at(ic, j, s0)] : T(0);
-        bc[q] = sv ? B[at(ic, j, s0)] : T(0);
-        bp[q] = T(0);
-        wm[q] = wc[q] = wn[q] = T(0);
-        yn[q] = zn[q] = bn[q] = T(0);
+    for (int q = 0; q < RY; ++q) {
+        dr[q] = miry(j0 + jr + q);
+        const int i = i0 + lx + dc, j = j0 + jr + q + dr[q];
+        val[q] = inxy(i, j);
+        to[q] = (first ? ybox(i, j) : val[q]) ? off(jr + q + dr[q], lx + dc) : kOob;
+        so[q] = inxy(i0 + lx, j0 + jr + q) ? off(jr + q, lx) : kOob;
     }
-    if (has1) {
-        qm = yld(i1, j1, s0 - 1);
-        qc = yld(i1, j1, s0);
-        qp = yld(i1, j1, s0 + 1);
-        if (solver(i1, j1, s0)) {
-            qz = Z[at(i1, j1, s0)];
-            qb = B[at(i1, j1, s0)];
+    // whether the tile or its rings hold a ghost in x or y (uniform)
+    const bool ghosts = NEU && (((cg.neu & 1) && i0 == g.lo0) || ((cg.neu & 2) && i0 + kTX + S > cg.hi_d[0]) ||
+                                ((cg.neu & 4) && j0 == g.lo1) || ((cg.neu & 8) && j0 + TY + S > cg.hi_d[1]));
+    // ring points: position, mirrored centre, validity
+    int pr[3] = {0, 0, 0}, pc[3] = {0, 0, 0}, mr[3], mc[3];
+    bool has[3], rv[3];
+    unsigned ro[3];
+#pragma unroll
+    for (int d = 0; d < S; ++d) {
+        has[d] = tid < NR[d];
+        if (has[d]) {
+            if (d == 0) ring_point<kTX, TY>(tid, pr[d], pc[d]);
+            else if (d == 1) ring_point<kTX + 2, TY + 2>(tid, pr[d], pc[d]);
+            else ring_point<kTX + 4, TY + 4>(tid, pr[d], pc[d]);
+            pr[d] -= d;
+            pc[d] -= d;
         }
+        mr[d] = pr[d] + miry(j0 + pr[d]);
+        mc[d] = pc[d] + mirx(i0 + pc[d]);
+        rv[d] = has[d] && inxy(i0 + mc[d], j0 + mr[d]);
+        ro[d] = has[d] && (first ? ybox(i0 + mc[d], j0 + mr[d]) : rv[d]) ? off(mr[d], mc[d]) : kOob;
     }
-    if (has2) oc = yld(i2, j2, s0);
 
-    for (int s = s0; s <= k1; ++s) {
-        const int buf = s & 1;
+    ChebPoint<T> t[RY], r[2];  // r[d]: ring d + 1 where it forms a level (d < S - 1)
+    T oc, on = T(0);           // outermost ring: Y of planes s, s + 1
+    auto zin = [&](int k) { return k >= g.lo2 && k < g.hi2; };
+    auto yin = [&](int k) { return first ? k >= 0 && k < cg.ng[2] : zin(k); };
+    const T* Yo = A.Y + org;
+    const T* Zo = first ? Yo : A.Z + org;
+    const T* Bo = A.B + org;
+    auto yrs = [&](int k) { return plane_rsrc(Yo + g.plane * k, yin(k)); };
+    auto zrs = [&](int k) { return plane_rsrc(Zo + g.plane * k, !first && zin(k)); };
+    auto brs = [&](int k) { return plane_rsrc(Bo + g.plane * k, !first && zin(k)); };
+    const int s0 = k0 - (S - 1), s1 = k1 + S - 2;  // steps s0 .. s1
+    {
+        const auto ya = yrs(s0 - 1), yb = yrs(s0), yc = yrs(s0 + 1), za = zrs(s0), ba = brs(s0);
+        auto start = [&](ChebPoint<T>& P, unsigned o) {
+            P = ChebPoint<T>{};
+            P.ym = buf_ld<T>(ya, o);
+            P.yc = buf_ld<T>(yb, o);
+            P.yp = buf_ld<T>(yc, o);
+            P.zc = buf_ld<T>(za, o);
+            P.bc = buf_ld<T>(ba, o);
+        };
+#pragma unroll
+        for (int q = 0; q < RY; ++q) start(t[q], to[q]);
+#pragma unroll
+        for (int d = 0; d < S - 1; ++d) start(r[d], ro[d]);
+        oc = buf_ld<T>(yb, ro[S - 1]);
+    }
+
+    for (int s = s0; s <= s1; ++s) {
+        const int buf = s & 1, alt = buf ^ 1;
         // Y of plane s into LDS
 #pragma unroll
-        for (int q = 0; q < kCpRY; ++q) ysl[buf][ly + kCpW * q + 2][lx + 2] = yc[q];
-        if (has1) ysl[buf][r1r + 1][r1c + 1] = qc;
-        if (has2) ysl[buf][r2r][r2c] = oc;
-        // loads for the next step: Y of plane s+2 (s+1 for the outer ring), Z and B of plane s+1
-        const bool ny = s + 2 <= k1 + 1, nzb = s + 1 <= k1;
+        for (int q = 0; q < RY; ++q) ysl[buf][jr + q + S][lx + S] = t[q].yc;
 #pragma unroll
-        for (int q = 0; q < kCpRY; ++q) {
-            const int j = j0 + ly + kCpW * q;
-            if (ny) yn[q] = yld(ic, j, s + 2);
-            const bool sv = nzb && solver(ic, j, s + 1);
-            zn[q] = sv ? Z[at(ic, j, s + 1)] : T(0);
-            bn[q] = sv ? B[at(ic, j, s + 1)] : T(0);
-        }
-        if (has1) {
-            if (ny) qn = yld(i1, j1, s + 2);
-            const bool sv = nzb && solver(i1, j1, s + 1);
-            qzn = sv ? Z[at(i1, j1, s + 1)] : T(0);
-            qbn = sv ? B[at(i1, j1, s + 1)] : T(0);
-        }
-        if (has2 && nzb) on = yld(i2, j2, s + 1);
-        __syncthreads();
-        // W1 of plane s on the tile and its ring (0 off the solver region)
-#pragma unroll
-        for (int q = 0; q < kCpRY; ++q) {
-            const int j = j0 + ly + kCpW * q;
-            const int r = ly + kCpW * q + 2, c = lx + 2;
-            T w = T(0);
-            if (solver(ic, j, s)) {
-                const T v = yc[q];
-                const T Av = cx * ((ysl[buf][r][c - 1] - v) + (ysl[buf][r][c + 1] - v)) +
-                             cy * ((ysl[buf][r - 1][c] - v) + (ysl[buf][r + 1][c] - v)) +
-                             czz * ((ym[q] - v) + (yp[q] - v));
-                w = a1 * v + b1 * (bc[q] + Av) - c1 * zc[q];
-                if constexpr (!LAST)
-                    if (s >= k0 && s < k1) put<NT>(W1 + at(ic, j, s), w);
-            }
-            wn[q] = w;
-            wsl[buf][r - 1][c - 1] = w;
-        }
-        if (has1) {
-            T w = T(0);
-            if (solver(i1, j1, s)) {
-                const int r = r1r + 1, c = r1c + 1;
-                const T v = qc;
-                const T Av = cx * ((ysl[buf][r][c - 1] - v) + (ysl[buf][r][c + 1] - v)) +
-                             cy * ((ysl[buf][r - 1][c] - v) + (ysl[buf][r + 1][c] - v)) +
-                             czz * ((qm - v) + (qp - v));
-                w = a1 * v + b1 * (qb + Av) - c1 * qz;
-            }
-            wsl[buf][r1r][r1c] = w;
-        }
-        __syncthreads();
-        // Neumann x/y ghosts of W1: the data point two cells inward
-        if (cg.neu & 15) {
-            const bool zin = s >= cg.lo_d[2] && s < cg.hi_d[2];
-            auto mirror = [&](int i, int j, int r, int c) {
-                if (!zin) return;
-                const bool yin = j >= cg.lo_d[1] && j < cg.hi_d[1], xin = i >= cg.lo_d[0] && i < cg.hi_d[0];
-                if ((cg.neu & 1) && i == cg.lo_d[0] - 1 && yin) wsl[buf][r][c] = wsl[buf][r][c + 2];
-                else if ((cg.neu & 2) && i == cg.hi_d[0] && yin) wsl[buf][r][c] = wsl[buf][r][c - 2];
-                else if ((cg.neu & 4) && j == cg.lo_d[1] - 1 && xin) wsl[buf][r][c] = wsl[buf][r + 2][c];
-                else if ((cg.neu & 8) && j == cg.hi_d[1] && xin) wsl[buf][r][c] = wsl[buf][r - 2][c];
+        for (int d = 0; d < S - 1; ++d)
+            if (has[d]) ysl[buf][pr[d] + S][pc[d] + S] = r[d].yc;
+        if (has[S - 1]) ysl[buf][pr[S - 1] + S][pc[S - 1] + S] = oc;
+        // loads for the next step: Y of plane s + 2 (s + 1 on the outermost ring), Z and B of plane s + 1
+        {
+            const auto y1 = plane_rsrc(Yo + g.plane * (s + 1), s < s1 && yin(s + 1));
+            const auto y2 = plane_rsrc(Yo + g.plane * (s + 2), s < s1 && yin(s + 2));
+            const auto z1 = plane_rsrc(Zo + g.plane * (s + 1), s < s1 && !first && zin(s + 1));
+            const auto b1 = plane_rsrc(Bo + g.plane * (s + 1), s < s1 && !first && zin(s + 1));
+            auto fetch = [&](ChebPoint<T>& P, unsigned o) {
+                P.yn = buf_ld<T>(y2, o);
+                P.zn = buf_ld<T>(z1, o);
+                P.bn = buf_ld<T>(b1, o);
             };
 #pragma unroll
-            for (int q = 0; q < kCpRY; ++q) mirror(ic, j0 + ly + kCpW * q, ly + kCpW * q + 1, lx + 1);
-            if (has1) mirror(i1, j1, r1r, r1c);
-        }
-        // W2 of plane s-1 on the tile (W1 of plane s-1 is in the other LDS buffer)
-        if (s - 1 >= k0) {
-            const int p = s - 1, pb = buf ^ 1;
-            const bool zlo = (cg.neu & 16) && p == cg.lo_d[2], zhi = (cg.neu & 32) && p == cg.hi_d[2] - 1;
+            for (int q = 0; q < RY; ++q) fetch(t[q], to[q]);
 #pragma unroll
-            for (int q = 0; q < kCpRY; ++q) {
-                const int j = j0 + ly + kCpW * q;
-                if (!solver(ic, j, p)) continue;
-                const int r = ly + kCpW * q + 1, c = lx + 1;
-                const T v = wc[q];
-                const T m = zlo ? wn[q] : wm[q];
-                const T u = zhi ? wm[q] : wn[q];
-                const T Av = cx * ((wsl[pb][r][c - 1] - v) + (wsl[pb][r][c + 1] - v)) +
-                             cy * ((wsl[pb][r - 1][c] - v) + (wsl[pb][r + 1][c] - v)) + czz * ((m - v) + (u - v));
-                const T w = a2 * v + b2 * (bp[q] + Av) - c2 * ym[q];
-                if constexpr (sizeof(TO) == sizeof(T)) put<NT>(W2 + at(ic, j, p), (TO)(sign < 0 ? -w : w));
-                else put<NT>(W2 + at(ic, j, p), (TO)(sign * (double)w));
+            for (int d = 0; d < S - 1; ++d) fetch(r[d], ro[d]);
+            on = buf_ld<T>(y1, ro[S - 1]);
+        }
+        __syncthreads();
+
+        // Neumann ghosts in z of the planes whose level is formed in this step: the
+        // register of the plane beyond the face takes the mirror plane's value
+        // (what it held belongs to a plane off the solver region, where every
+        // level is 0)
+        if constexpr (NEU) {
+            const int lo = cg.lo_d[2], hi = cg.hi_d[2] - 1;
+            auto each = [&](auto f) {
+#pragma unroll
+                for (int q = 0; q < RY; ++q) f(t[q]);
+#pragma unroll
+                for (int d = 0; d < S - 1; ++d) f(r[d]);
+            };
+            if ((cg.neu & 16) && s == lo) each([](ChebPoint<T>& P) { P.ym = P.yp; });
+            if ((cg.neu & 32) && s == hi) each([](ChebPoint<T>& P) { P.yp = P.ym; });
+        }
+        // level 1 of plane s
+        {
+            const bool zs = zin(s);
+            auto level1 = [&](ChebPoint<T>& P, T Av) {
+                if (first) {
+                    P.bc = P.yc;
+                    return cheb_start(A.c1, A.c0, P.yc, Av);
+                }
+                return cheb_level(A.a[0], P.yc, A.b[0], P.bc, Av, A.c[0], P.zc);
+            };
+            auto at = [&](const ChebPoint<T>& P, int row, int col) {
+                const T(*y)[kTX + 2 * S] = ysl[buf];
+                return lap7(P.yc, y[row][col - 1], y[row][col + 1], y[row - 1][col], y[row + 1][col], P.ym, P.yp, cx, cy, cz);
+            };
+            T Av[RY];
+            if (!NEU || !ghosts) {
+#pragma unroll
+                for (int q = 0; q < RY; ++q) {
+                    const int row = jr + q + S, col = lx + S;
+                    const T ym = q > 0 ? t[q > 0 ? q - 1 : 0].yc : ysl[buf][row - 1][col];
+                    const T yp = q + 1 < RY ? t[q + 1 < RY ? q + 1 : 0].yc : ysl[buf][row + 1][col];
+                    Av[q] = lap7(t[q].yc, ysl[buf][row][col - 1], ysl[buf][row][col + 1], ym, yp, t[q].ym, t[q].yp, cx, cy, cz);
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < RY; ++q) Av[q] = at(t[q], jr + q + dr[q] + S, lx + dc + S);
+            }
+            const auto wr = plane_rsrc((A.Wp ? A.Wp : (T*)A.Y) + org + g.plane * s, S == 2 && A.Wp && s >= k0 && s < k1);
+#pragma unroll
+            for (int q = 0; q < RY; ++q) {
+                T w = level1(t[q], Av[q]);
+                if (!(val[q] && zs)) w = T(0);
+                t[q].un = w;
+                usl[buf][jr + q + S - 1][lx + S - 1] = w;
+                if constexpr (S == 2) buf_st<NT>(wr, so[q], w);
+            }
+#pragma unroll
+            for (int d = 0; d < S - 1; ++d) {
+                if (!has[d]) continue;
+                T w = level1(r[d], at(r[d], mr[d] + S, mc[d] + S));
+                if (!(rv[d] && zs)) w = T(0);
+                r[d].un = w;
+                usl[buf][pr[d] + S - 1][pc[d] + S - 1] = w;
+            }
+        }
+        // level 2 of plane s - 1 (level 1 of that plane is in the other LDS buffer)
+        if (s >= s0 + 2) {
+            const int p = s - 1;
+            const bool zs = zin(p), own = p >= k0 && p < k1;
+            if constexpr (NEU) {
+                const bool zlo = (cg.neu & 16) && p == cg.lo_d[2], zhi = (cg.neu & 32) && p == cg.hi_d[2] - 1;
+                auto mirror = [&](ChebPoint<T>& P) {
+                    if (zlo) P.um = P.un;
+                    else P.un = P.um;
+                };
+                if (zlo || zhi) {
+#pragma unroll
+                    for (int q = 0; q < RY; ++q) mirror(t[q]);
+                    if constexpr (S == 3) mirror(r[0]);
+                }
+            }
+            auto level2 = [&](const ChebPoint<T>& P, T Av) {
+                return cheb_level(A.a[1], P.uc, A.b[1], P.b1, Av, A.c[1], first ? A.c0 * P.ym : P.ym);
+            };
+            auto at = [&](const ChebPoint<T>& P, int row, int col) {
+                const T(*u)[kTX + 2 * (S - 1)] = usl[alt];
+                return lap7(P.uc, u[row][col - 1], u[row][col + 1], u[row - 1][col], u[row + 1][col], P.um, P.un, cx, cy, cz);
+            };
+            T Av[RY];
+            if (!NEU || !ghosts) {
+#pragma unroll
+                for (int q = 0; q < RY; ++q) {
+                    const int row = jr + q + S - 1, col = lx + S - 1;
+                    const T ym = q > 0 ? t[q > 0 ? q - 1 : 0].uc : usl[alt][row - 1][col];
+                    const T yp = q + 1 < RY ? t[q + 1 < RY ? q + 1 : 0].uc : usl[alt][row + 1][col];
+                    Av[q] = lap7(t[q].uc, usl[alt][row][col - 1], usl[alt][row][col + 1], ym, yp, t[q].um, t[q].un, cx, cy, cz);
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < RY; ++q) Av[q] = at(t[q], jr + q + dr[q] + S - 1, lx + dc + S - 1);
+            }
+            const auto wr = plane_rsrc((A.Wp ? A.Wp : (T*)A.Y) + org + g.plane * p, S == 3 && A.Wp && own);
+            const auto xr = plane_rsrc(A.W + org + g.plane * p, S == 2 && own);
+#pragma unroll
+            for (int q = 0; q < RY; ++q) {
+                T w = level2(t[q], Av[q]);
+                if constexpr (S == 2) {
+                    buf_st<NT>(xr, so[q] == kOob ? kOob : so[q] * (unsigned)(sizeof(TO) / sizeof(T)), (TO)(A.sign * w));
+                } else {
+                    if (!(val[q] && zs)) w = T(0);
+                    t[q].vn = w;
+                    vsl[alt][jr + q + 1][lx + 1] = w;
+                    buf_st<NT>(wr, so[q], w);
+                }
+            }
+            if constexpr (S == 3) {
+                if (has[0]) {
+                    T w = level2(r[0], at(r[0], mr[0] + S - 1, mc[0] + S - 1));
+                    if (!(rv[0] && zs)) w = T(0);
+                    vsl[alt][pr[0] + 1][pc[0] + 1] = w;
+                }
+            }
+        }
+        // level 3 of plane s - 2
+        if constexpr (S == 3) {
+            if (s >= s0 + 4) {
+                const int p = s - 2;
+                if constexpr (NEU) {
+                    const bool zlo = (cg.neu & 16) && p == cg.lo_d[2], zhi = (cg.neu & 32) && p == cg.hi_d[2] - 1;
+                    if (zlo || zhi) {
+#pragma unroll
+                        for (int q = 0; q < RY; ++q) {
+                            if (zlo) t[q].vm = t[q].vn;
+                            else t[q].vn = t[q].vm;
+                        }
+                    }
+                }
+                const auto xr = plane_rsrc(A.W + org + g.plane * p, true);
+#pragma unroll
+                for (int q = 0; q < RY; ++q) {
+                    const int row = jr + q + 1, col = lx + 1;
+                    const T ym = q > 0 ? t[q > 0 ? q - 1 : 0].vc : vsl[buf][row - 1][col];
+                    const T yp = q + 1 < RY ? t[q + 1 < RY ? q + 1 : 0].vc : vsl[buf][row + 1][col];
+                    const T Av = lap7(t[q].vc, vsl[buf][row][col - 1], vsl[buf][row][col + 1], ym, yp, t[q].vm, t[q].vn, cx,
+                                      cy, cz);
+                    const T w = cheb_level(A.a[2], t[q].vc, A.b[2], t[q].b2, Av, A.c[2], t[q].um);
+                    buf_st<NT>(xr, so[q] == kOob ? kOob : so[q] * (unsigned)(sizeof(TO) / sizeof(T)), (TO)(A.sign * w));
+                }
             }
         }
         // advance one plane
+        auto step = [&](ChebPoint<T>& P) {
+            P.ym = P.yc;
+            P.yc = P.yp;
+            P.yp = P.yn;
+            P.zc = P.zn;
+            P.b2 = P.b1;
+            P.b1 = P.bc;
+            P.bc = P.bn;
+            P.um = P.uc;
+            P.uc = P.un;
+            P.vm = P.vc;
+            P.vc = P.vn;
+        };
 #pragma unroll
-        for (int q = 0; q < kCpRY; ++q) {
-            ym[q] = yc[q];
-            yc[q] = yp[q];
-            yp[q] = yn[q];
-            zc[q] = zn[q];
-            bp[q] = bc[q];
-            bc[q] = bn[q];
-            wm[q] = wc[q];
-            wc[q] = wn[q];
-        }
-        qm = qc;
-        qc = qp;
-        qp = qn;
-        qz = qzn;
-        qb = qbn;
+        for (int q = 0; q < RY; ++q) step(t[q]);
+#pragma unroll
+        for (int d = 0; d < S - 1; ++d) step(r[d]);
         oc = on;
     }
 }
 
-template <typename T, typename TO>
-void launch_cheb_pair(const Geo& g0, const ChebPairGeo& cg, hipStream_t s, const T* Y, const T* Z, const T* B, T* W1,
-                      TO* W2, const double a[2], const double b[2], const double c[2], double sign, bool last,
-                      const int* gate)
+template <typename T, typename TO, int S, int RY>
+static void run_cheb_multi(const Geo& g0, const ChebPairGeo& cg, hipStream_t s, const ChebArgs<T, TO>& A, int slots)
 {
-    Geo g = g0;
-    g.ntx = (g.hi0 - g.lo0 + kTX - 1) / kTX;
-    g.nty = (g.hi1 - g.lo1 + kCpTY - 1) / kCpTY;
-    // z-chunk: as set, or the longest of 64, 32, 16 planes giving 1024 blocks
-    // (two rounds of the two blocks per CU that fit; halo planes cost 2 / kz)
-    const int nz = g.hi2 - g.lo2;
-    g.kz = cg.kz;
-    if (g.kz <= 0) {
-        g.kz = 64;
-        while (g.kz > 16 && (long long)g.ntx * g.nty * ((nz + g.kz - 1) / g.kz) < 1024) g.kz /= 2;
+    constexpr int TY = kChW * RY;
+    const int nx = g0.hi0 - g0.lo0, ny = g0.hi1 - g0.lo1, nz = g0.hi2 - g0.lo2;
+    const long long tiles = (long long)((nx + kTX - 1) / kTX) * ((ny + TY - 1) / TY);
+    const Geo g = retile(g0, TY, cg.kz > 0 ? cg.kz : pick_kz(tiles, nz, slots, 2 * S));
+    const dim3 grid(g.nblocks), block(kTX, kChW);
+    if (cg.neu && g.nt) hipLaunchKernelGGL((k_cheb_multi<T, TO, S, RY, true, true>), grid, block, 0, s, g, cg, A);
+    else if (cg.neu) hipLaunchKernelGGL((k_cheb_multi<T, TO, S, RY, true, false>), grid, block, 0, s, g, cg, A);
+    else if (g.nt) hipLaunchKernelGGL((k_cheb_multi<T, TO, S, RY, false, true>), grid, block, 0, s, g, cg, A);
+    else hipLaunchKernelGGL((k_cheb_multi<T, TO, S, RY, false, false>), grid, block, 0, s, g, cg, A);
+}
+
+template <typename T, typename TO>
+void launch_cheb_multi(const Geo& g, const ChebPairGeo& cg, hipStream_t s, int sweeps, const T* Y, const T* Z, const T* B,
+                       T* Wp, TO* W, const double* a, const double* b, const double* c, double c0, double c1, double sign,
+                       const int* gate)
+{
+    if (g.hi0 <= g.lo0 || g.hi1 <= g.lo1 || g.hi2 <= g.lo2) return;
+    ChebArgs<T, TO> A{};
+    A.Y = Y;
+    A.Z = Z;
+    A.B = B;
+    A.Wp = Wp;
+    A.W = W;
+    for (int l = 0; l < sweeps; ++l) {
+        A.a[l] = (T)a[l];
+        A.b[l] = (T)b[l];
+        A.c[l] = (T)c[l];
     }
-    const int ntz = (nz + g.kz - 1) / g.kz;
-    const long long nb = (long long)g.ntx * g.nty * ntz;
-    if (g.ntx <= 0 || g.nty <= 0 || ntz <= 0) return;
-    if (nb > 0x7FFFFFFFll) {
-        std::fprintf(stderr, "pps: fused Chebyshev grid too large; launch skipped\n");
-        return;
-    }
-    const dim3 grid((unsigned)nb), block(kTX, kCpW);
-    const T A1 = (T)a[0], B1 = (T)b[0], C1 = (T)c[0], A2 = (T)a[1], B2 = (T)b[1], C2 = (T)c[1];
-    if (last) {
-        if (g.nt) hipLaunchKernelGGL((k_cheb_pair<T, TO, true, true>), grid, block, 0, s, g, cg, Y, Z, B, W1, W2, A1, B1, C1, A2, B2, C2, sign, gate);
-        else hipLaunchKernelGGL((k_cheb_pair<T, TO, false, true>), grid, block, 0, s, g, cg, Y, Z, B, W1, W2, A1, B1, C1, A2, B2, C2, sign, gate);
-    } else if constexpr (std::is_same_v<T, TO>) {
-        if (g.nt) hipLaunchKernelGGL((k_cheb_pair<T, T, true, false>), grid, block, 0, s, g, cg, Y, Z, B, W1, W2, A1, B1, C1, A2, B2, C2, sign, gate);
-        else hipLaunchKernelGGL((k_cheb_pair<T, T, false, false>), grid, block, 0, s, g, cg, Y, Z, B, W1, W2, A1, B1, C1, A2, B2, C2, sign, gate);
-    } else {
-        std::fprintf(stderr, "pps: a fused Chebyshev pair changes precision only on its last output; launch skipped\n");
-    }
+    A.c0 = (T)c0;
+    A.c1 = (T)c1;
+    A.sign = (T)sign;
+    A.gate = gate;
+    // 32-row tiles read fewer ring points (one block per CU); 16-row tiles (two per
+    // CU; one with Neumann faces, whose FP64 form for three sweeps needs more
+    // registers) where the 32-row ones do not give every CU 8 planes of work or
+    // where the last row of tiles is at most half full.  us per BiCGSTAB +
+    // Chebyshev(24) iteration, 32 / 16 rows: Dirichlet 130^3 621 / 573, 194^3
+    // 1461 / 1503, 514^3 24500 / 24730; mixed faces 130^3 (129 rows) 807 / 762,
+    // 131x257x190 (256 rows) 1796 / 1859, 258^3 (257 rows) 4334 / 3997
+    const int nx = g.hi0 - g.lo0, ny = g.hi1 - g.lo1, nz = g.hi2 - g.lo2, tail = (ny - 1) % (4 * kChW) + 1;
+    const long long tiles = (long long)((nx + kTX - 1) / kTX) * ((ny + 4 * kChW - 1) / (4 * kChW));
+    const bool tall = tiles * nz >= 8ll * kCUs && tail > 2 * kChW;
+    if (sweeps == 3 && tall) run_cheb_multi<T, TO, 3, 4>(g, cg, s, A, kCUs);
+    else if (sweeps == 3) run_cheb_multi<T, TO, 3, 2>(g, cg, s, A, cg.neu && sizeof(T) == 8 ? kCUs : 2 * kCUs);
+    else if (tall) run_cheb_multi<T, TO, 2, 4>(g, cg, s, A, kCUs);
+    else run_cheb_multi<T, TO, 2, 2>(g, cg, s, A, 2 * kCUs);
 }
 
 // ------------------------------------------------------------------ FCG
@@ -2479,15 +2670,13 @@ void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, floa
 PPS_INST_T(double)
 PPS_INST_T(float)
 
-template void launch_cheb_pair<double, double>(const Geo&, const ChebPairGeo&, hipStream_t, const double*,
-                                               const double*, const double*, double*, double*, const double[2],
-                                               const double[2], const double[2], double, bool, const int*);
-template void launch_cheb_pair<float, float>(const Geo&, const ChebPairGeo&, hipStream_t, const float*, const float*,
-                                             const float*, float*, float*, const double[2], const double[2],
-                                             const double[2], double, bool, const int*);
-template void launch_cheb_pair<float, double>(const Geo&, const ChebPairGeo&, hipStream_t, const float*, const float*,
-                                              const float*, float*, double*, const double[2], const double[2],
-                                              const double[2], double, bool, const int*);
+#define PPS_INST_CHEB(T, TO)                                                                                     \
+    template void launch_cheb_multi<T, TO>(const Geo&, const ChebPairGeo&, hipStream_t, int, const T*, const T*,  \
+                                           const T*, T*, TO*, const double*, const double*, const double*, double, \
+                                           double, double, const int*);
+PPS_INST_CHEB(double, double)
+PPS_INST_CHEB(float, float)
+PPS_INST_CHEB(float, double)
 template void launch_cheb_sweep<double, double>(const Geo&, hipStream_t, const double*, const double*, const double*,
                                                 double*, double, double, double, double, const int*);
 template void launch_cheb_sweep<float, float>(const Geo&, hipStream_t, const float*, const float*, const float*, float*,

@@ -223,20 +223,25 @@ void launch_cheb_first(const Geo& g, hipStream_t s, const T* B, T* Z, T* Y, doub
 template <typename T, typename TO>
 void launch_cheb_sweep(const Geo& g, hipStream_t s, const T* Y, const T* B, const T* Z, TO* W, double a, double b,
                        double c, double sign, const int* gate);
-// X = sign*c0*B (degree-0/1 outputs) and X = sign*c1*(2B + c0*AB)
-// two fused sweeps (c, c+1) of the Chebyshev recurrence: W1 = y_{c+1} (not
-// written when `last`), W2 = y_{c+2} (sign-applied and converted to TO when
-// `last`, the stage output).  Y = y_c needs its Neumann ghosts set; Z = y_{c-1}.
+// geometry of the fused Chebyshev sweeps
 struct ChebPairGeo {
     int lo_d[3], hi_d[3];  // data region (the Neumann ghosts' mirror rule)
-    int ng[3];             // guarded box (loads outside it read 0)
+    int ng[3];             // guarded box
     int neu;               // bit f set: face f (x- x+ y- y+ z- z+) is Neumann
     int kz;                // z-chunk of one block
 };
+// `sweeps` = 2 or 3 fused sweeps: W = the last one's y (sign-applied and
+// converted to TO), Wp = the one before (null: not written).  Y = y_c and
+// Z = y_{c-1}; Z = null: the recurrence's start, Y = B, whose first level is
+// c1 (2B + c0 AB) (a[0], b[0], c[0] unused; B's values off the solver region
+// take part, its Neumann ghosts must be set).  Otherwise nothing is read off the
+// solver region: the levels' Neumann ghosts are formed in the kernel, their
+// other points there count as 0.  40 rows of a field must be smaller than 2 GiB.
 template <typename T, typename TO>
-void launch_cheb_pair(const Geo& g, const ChebPairGeo& cg, hipStream_t s, const T* Y, const T* Z, const T* B, T* W1,
-                      TO* W2, const double a[2], const double b[2], const double c[2], double sign, bool last,
-                      const int* gate);
+void launch_cheb_multi(const Geo& g, const ChebPairGeo& cg, hipStream_t s, int sweeps, const T* Y, const T* Z, const T* B,
+                       T* Wp, TO* W, const double* a, const double* b, const double* c, double c0, double c1, double sign,
+                       const int* gate);
+// X = sign*c0*B (degree-0/1 outputs) and X = sign*c1*(2B + c0*AB)
 template <typename T, typename TO>
 void launch_cheb_first_out(const Geo& g, hipStream_t s, const T* B, TO* X, double c0, double c1, int which,
                            double sign, const int* gate);
