@@ -1551,7 +1551,9 @@ int pps_create(const pps_grid* grid, void** out)
     const long long nvec = (long long)((X.ng[0] + kThreads - 1) / kThreads) * X.ng[1] * X.ng[2];
     // one-plane chunks of 64 x 16 tiles (small grids' CG pass)
     const long long nsmall = (long long)((X.ng[0] + kTX - 1) / kTX) * ((X.ng[1] + 15) / 16) * X.ng[2];
-    X.rb.cap = (int)std::max(std::max<long long>(gbig.nblocks, nvec), nsmall) + 8;
+    // the network's output kernel: 14 x 18 tiles in chunks of 2 planes at least
+    const long long nout = (long long)((X.ng[0] + 13) / 14) * ((X.ng[1] + 17) / 18) * ((X.ng[2] + 1) / 2);
+    X.rb.cap = (int)std::max(std::max<long long>(gbig.nblocks, nvec), std::max(nsmall, nout)) + 8;
     X.rb.cap2 = X.rb.cap / kSpan + 8;
     rc = rc ? rc : X.hip(hipMalloc(&X.rb.partials2, sizeof(double) * kMaxRedQ * X.rb.cap2), "span partials");
     // a solve streams 4-8 fields per iteration: once a field passes 32 MiB
@@ -1918,8 +1920,11 @@ int pps_residual_noalloc(const pps_grid* grid, const double* x, const double* b,
     L.ox = 0;
     L.plane = (long long)L.ng[0] * L.ng[1];
     L.total = L.plane * L.ng[2];
-    // z-chunk: 16 planes, longer when a launch would need more blocks than
-    // the scratch holds partials
+    // z-chunk: 4 planes, 2 where those leave the chip short of blocks, longer
+    // when a launch would need more blocks than the scratch holds partials.  us at
+    // 2 / 4 / 16 planes: 67x45x130 8.8 / 10.0 / 25.0, 130^3 12.8 / 13.2 / 23.3,
+    // 322^3 155 / 146 / 146, 514^3 684 / 650 / 744 (the rows of this layout start
+    // anywhere in a cache line; short chunks keep neighbouring tiles close in time)
     const long long tiles = (long long)((R.hi[0] - R.lo[0] + kTX - 1) / kTX) * ((R.hi[1] - R.lo[1] + kTH - 1) / kTH);
     if (tiles > kScratchPartials) {
         g_create_error = "pps_residual_noalloc: an x-y plane needs more than 131072 tiles of " + std::to_string(kTX) +
@@ -1927,14 +1932,16 @@ int pps_residual_noalloc(const pps_grid* grid, const double* x, const double* b,
         return PPS_ERR_UNSUPPORTED;
     }
     const int nz = R.hi[2] - R.lo[2];
-    int kz = 16;
+    int kz = tiles * ((nz + 3) / 4) < 1024 ? 2 : 4;
     while (tiles * ((nz + kz - 1) / kz) > kScratchPartials) kz *= 2;
     double* sp = nullptr;
     int rc = scratch_for_current_device(&sp, g_create_error);
     if (rc) return rc;
     RedBuf rb{sp, nullptr, kScratchPartials};
     double* out = norm_dev ? norm_dev : sp + kScratchPartials;  // else the result slot past the partials
-    const Geo g = make_geo(L, R, coef, kz, (L.total * 8 > (32ll << 20)) ? 1 : 0);
+    // non-temporal stores once the three fields exceed the last-level cache:
+    // 272x370x51 (124 MB) 34 us with them, 28 without; 258^3 (422 MB) 76 / 85
+    const Geo g = make_geo(L, R, coef, kz, (L.total * 24 > (256ll << 20)) ? 1 : 0);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (launch_residual_norm(g, s, rb, x, b, r, out) != 0) {
         g_create_error = "pps_residual_noalloc: launch exceeds the scratch partials";

@@ -503,13 +503,15 @@ static bool check_capacity(const Geo& g, const RedBuf& rb)
 
 // tiling of a stencil launch: the z-chunk set on the context, or (kz_st = 0)
 // the longest of 64, 32, 16, 8 planes that still gives 2048 blocks (a longer
-// chunk re-reads fewer halo planes; 2048 blocks keep every CU busy to the end)
+// chunk re-reads fewer halo planes; 2048 blocks keep every CU busy to the end);
+// below 1024 blocks of 8 planes, 4 or 2 planes (a small grid's time is the
+// planes that one block marches through)
 static Geo stencil_geo(const Geo& g0)
 {
     if (g0.kz_st > 0) return retile(g0, kTH, g0.kz_st);
     int kz = 64;
     Geo g = retile(g0, kTH, kz);
-    while (kz > 8 && g.nblocks < 2048) {
+    while ((kz > 8 && g.nblocks < 2048) || (kz > 2 && g.nblocks < 1024)) {
         kz /= 2;
         g = retile(g0, kTH, kz);
     }

@@ -1112,17 +1112,6 @@ __global__ __launch_bounds__(kWThreads) __attribute__((amdgpu_waves_per_eu(4, 4)
     else run(std::false_type{});
 }
 
-// z-chunk of the wide-tile lift: at least 2048 blocks (4 per CU), chunks of
-// at least 16 planes, starting on even planes
-static int pick_zc_w(int D, int H, int W, int B)
-{
-    const long long tiles = (long long)((W + kWX - 1) / kWX) * ((H + kWY - 1) / kWY) * B;
-    int zc = D;
-    while (zc > 16 && tiles * ((D + zc - 1) / zc) < 2048) zc = (zc + 1) / 2;
-    if ((zc & 1) && zc < D) ++zc;
-    return std::max(zc, 1);
-}
-
 // z-chunk: enough blocks to fill the chip, at most one chunk per 16 planes
 static int pick_zc(int D, int H, int W, int B)
 {
@@ -1132,12 +1121,6 @@ static int pick_zc(int D, int H, int W, int B)
     if ((zc & 1) && zc < D) ++zc;  // chunks start on even planes (z pairs of the pooled lift output)
     return std::max(zc, 1);
 }
-// z-chunk of the forward convolutions.  Three blocks per CU are resident;
-// when a level's tiles fit one such round but pick_zc's chunks make more
-// blocks than that, the fewest chunks that fill one round run instead (fewer
-// halo planes, no partly filled last round: 512^3's level-1 layers 5-8 %
-// faster with 86-plane chunks than with 16).  Smaller launches keep pick_zc's
-// chunks (at level 2 of 512^3, 512 blocks of 16 planes beat 704 of 12).
 static int cu_count()
 {
     static int n = 0;
@@ -1151,6 +1134,30 @@ static int cu_count()
     }
     return n;
 }
+// z-chunk of the forward kernels that march z: the even one (or all of D) with
+// the least work for the busiest CU, blocks per CU times the chunk and its three
+// planes of prologue and halo.  A CU with fewer than `fill` blocks does not run
+// them faster, so fewer count as `fill`.  `keep` (or 0) is a chunk that was tuned
+// on large grids, kept unless the model promises 15 % (at 384^3 the model's choice
+// for level 1 is 3 % slower).  No result depends on the chunk (the output kernel's
+// partials of z . dot aside).  us per launch, chunks of 16 planes (the least there
+// was) / as picked: level 2 of 256^3 16.5 / 7.8 (2 planes); level 1 of 128^3 16.6 /
+// 8.0 (2); lift at 128^3 20.4 / 12.4 (4); output kernel at 64^3 20.6 / 11.7 (2), at
+// 256^3 155 / 145 (32)
+static int pick_zc_fill(long long tiles, int D, int fill, int keep)
+{
+    auto cost = [&](int c) {
+        const long long per_cu = (tiles * ((D + c - 1) / c) + cu_count() - 1) / cu_count();
+        return std::max<long long>(per_cu, fill) * (c + 3);
+    };
+    int best = std::min(2, D);
+    for (int zc = 4; zc <= 128 && zc < D + 2; zc += 2)
+        if (cost(std::min(zc, D)) <= cost(best)) best = std::min(zc, D);
+    return keep > 0 && 100 * cost(best) > 85 * cost(keep) ? keep : best;
+}
+// forward convolutions, three resident blocks per CU.  Where a level's tiles fit
+// one round of those but chunks of pick_zc make more blocks, the fewest chunks
+// that fill the round (level 1 of 512^3: 86 planes, 5-8 % faster than 16)
 static int pick_zc_conv(int D, int H, int W, int B)
 {
     int zc = pick_zc(D, H, W, B);
@@ -1161,7 +1168,17 @@ static int pick_zc_conv(int D, int H, int W, int B)
         zc = (int)((D + nz - 1) / nz);
         if ((zc & 1) && zc < D) ++zc;  // chunks start on even planes
     }
-    return zc;
+    return pick_zc_fill(tiles, D, 3, zc);
+}
+// wide-tile lift, two resident blocks per CU; on large grids at least 2048 blocks
+// in chunks of 16 planes or more
+static int pick_zc_w(int D, int H, int W, int B)
+{
+    const long long tiles = (long long)((W + kWX - 1) / kWX) * ((H + kWY - 1) / kWY) * B;
+    int zc = D;
+    while (zc > 16 && tiles * ((D + zc - 1) / zc) < 2048) zc = (zc + 1) / 2;
+    if ((zc & 1) && zc < D) ++zc;
+    return pick_zc_fill(tiles, D, 2, zc);
 }
 static dim3 conv_grid(int D, int H, int W, int B, int zc)
 {
@@ -1524,16 +1541,12 @@ __global__ __launch_bounds__(256, 4) void k_outf(ConvArgs a, int zc)
     }
 }
 
-// grid of the fused output kernel: 14 x 18 tiles, z-chunks so that the launch
-// has at least 8192 blocks (chunks of 16 planes or more)
+// grid of the fused output kernel: 14 x 18 tiles, four resident blocks per CU
 static dim3 outf_grid(int D, int H, int W, int* zc)
 {
-    const int tiles = ((W + kFW - 1) / kFW) * ((H + kFH - 1) / kFH);
-    int c = D;
-    while (c > 16 && (long long)tiles * ((D + c - 1) / c) < 8192) c = (c + 1) / 2;
-    if ((c & 1) && c < D) ++c;  // chunks start on even planes
-    *zc = c;
-    return dim3((unsigned)((W + kFW - 1) / kFW), (unsigned)((H + kFH - 1) / kFH), (unsigned)((D + c - 1) / c));
+    const int tx = (W + kFW - 1) / kFW, ty = (H + kFH - 1) / kFH;
+    *zc = pick_zc_fill((long long)tx * ty, D, 4, 0);
+    return dim3((unsigned)tx, (unsigned)ty, (unsigned)((D + *zc - 1) / *zc));
 }
 
 static long long outf_blocks(int D, int H, int W)
