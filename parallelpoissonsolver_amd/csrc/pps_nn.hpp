@@ -128,7 +128,7 @@ struct BufSet {
     bool train = false;
     int dims[3][3] = {};          // per level: D, H, W
     std::vector<uint16_t*> act, dact;
-    uint16_t* dx[3] = {nullptr, nullptr, nullptr};  // backward-data scratch per level
+    uint16_t* dx[3] = {nullptr, nullptr, nullptr};  // backward-data scratch of the pooled inputs (levels 1, 2)
     std::vector<uint16_t*> pooled;                  // pool(act i), written by act i's producer (or null)
     float *in = nullptr, *y = nullptr, *dy = nullptr, *ky = nullptr;
     double *g = nullptr, *lpart = nullptr, *coef = nullptr, *lossv = nullptr;
