@@ -1,8 +1,14 @@
 """The weight-gradient kernel at the edges of its 16 x 16 tiles and z-chunks:
 odd extents, one voxel past a tile, single planes at the coarsest level, and a
-depth of several chunks.  Against the numpy oracle with the bars of the network's
-gradient test: 3 % relative L2 per layer plus half the distance between the
-oracle's rounded and exact gradients (what BF16 storage alone moves).
+depth of several chunks.
+
+The oracle's backward pass runs on the activations and the output that the GPU
+itself stored, so both sides use the same inputs and the same ReLU masks; what
+is left are the stored BF16 gradients, each of which may round one ulp (2^-8 at
+most) apart where the FP32 sums differ.  A layer whose gradients all did so
+would be off by 2^-8 in relative L2; over the 13 layers that precede the first
+one, in quadrature, sqrt(13) 2^-8 = 1.4 %: the bar is 1.5 % per layer, where a
+lost row, plane or chunk of these extents is at least 2.5 % of the voxels.
 """
 import numpy as np
 import pytest
@@ -10,6 +16,39 @@ import pytest
 from oracle import nn_oracle as O
 
 pytestmark = pytest.mark.gpu
+
+
+def backward(p, x, y, acts, g):
+    """Gradient of every stored parameter, rounded where the GPU rounds, from given activations."""
+    f = np.float32
+    weights = O._weights(p, True)
+    _, dy = O.loss_and_dy(y, x, g)
+    dy = dy.astype(f)
+    grad, dacts = [None] * O.N_LAYERS, [None] * len(acts)
+    for l in range(O.N_LAYERS - 1, -1, -1):
+        cin, cout, _, mode, ia, sk, _ = O.NET[l]
+        xin = O._layer_input(l, x, acts, True).astype(f)
+        if l == O.N_LAYERS - 1:
+            dz = np.zeros(dy.shape + (O.C,), f)
+            dz[..., 0] = O.bf16(dy)
+        else:
+            dz = np.where(acts[l] > 0, dacts[l], 0).astype(f)
+        w = O.conv_dw(xin, dz)
+        b = dz.astype(np.float64).sum(axis=(0, 1, 2, 3))
+        w[:, cin:, :] = 0
+        w[:, :, cout:] = 0
+        b[cout:] = 0
+        grad[l] = np.concatenate([w.reshape(-1), b])
+        if l == 0:
+            return grad
+        dx = O.bf16(O.conv(dz, O.flip_transpose(weights[l][0]).astype(f)).astype(f))
+        if mode == "plain":
+            dacts[ia] = dx
+        elif mode == "pool":
+            dacts[ia] = O.bf16(dacts[ia] + O.pool_back(dx, acts[ia].shape[1:4]))
+        else:
+            dacts[sk] = dx
+            dacts[ia] = O.bf16(O.up_back(dx, acts[ia].shape[1:4]))
 
 
 @pytest.mark.parametrize("shape", [(1, 3, 2, 5), (2, 5, 17, 16), (1, 33, 15, 34), (1, 40, 33, 9)])
@@ -24,12 +63,10 @@ def test_weight_gradient_edges(shape):
     p = net.get_params()
     x = rng.normal(size=shape).astype(np.float32)
     g = rng.uniform(1.0, 3.0, shape[0])
-    loss, grad = net.loss_grad(x, g)
-    lo, go = O.loss_grad(p, x, g, rounding=True)
-    _, gx = O.loss_grad(p.astype(np.float64), x.astype(np.float64), g, rounding=False)
-    assert abs(loss - lo) < 1e-3 * max(1.0, abs(lo))
+    y = net.forward(x)
+    _, grad = net.loss_grad(x, g)
+    ref = backward(p, x, y, [net.activation(i) for i in range(O.N_LAYERS - 1)], g)
     for l in range(O.N_LAYERS):
-        sl = slice(l * O.LAYER_PARAMS, (l + 1) * O.LAYER_PARAMS)
-        bf16_effect = np.linalg.norm(go[sl] - gx[sl])
-        assert np.linalg.norm(grad[sl] - go[sl]) <= 3e-2 * np.linalg.norm(go[sl]) + 0.5 * bf16_effect + 1e-9, l
+        got = grad[l * O.LAYER_PARAMS:(l + 1) * O.LAYER_PARAMS]
+        assert np.linalg.norm(got - ref[l]) <= 1.5e-2 * np.linalg.norm(ref[l]), l
     net.close()
