@@ -66,6 +66,9 @@ struct Stage {
     virtual long long iters_per_call() const { return 0; }
     // operator()(out, in) as a preconditioner; kernels gated on *gate
     virtual int apply(Field out, Field in, const int* gate) = 0;
+    // apply() for a caller that does not read `in`'s Neumann ghosts afterwards:
+    // they need not be reset in place
+    virtual int apply_internal(Field out, Field in, const int* gate) { return apply(out, in, gate); }
     // apply() that may also sum out . dot into the context's reduction
     // partials: *nblocks = their count, or 0 when the stage does not
     virtual int apply_dot(Field out, Field in, const int* gate, Field dot, int* nblocks)
@@ -146,6 +149,13 @@ struct Ctx {
     Geo gsolver(int prec) const { return geo(solver, prec); }
     Geo gbox(int prec) const { return geo(box, prec); }
     Geo gdata(int prec) const { return geo(data, prec); }
+    int neumann() const
+    {
+        int m = 0;
+        for (int f = 0; f < 6; ++f)
+            if (grid.bcs_type[f] == 1) m |= 1 << f;
+        return m;
+    }
     ChebPairGeo cheb_pair_geo() const
     {
         ChebPairGeo cg{};
@@ -154,8 +164,7 @@ struct Ctx {
             cg.hi_d[d] = lim_data[2 * d + 1];
             cg.ng[d] = ng[d];
         }
-        for (int f = 0; f < 6; ++f)
-            if (grid.bcs_type[f] == 1) cg.neu |= 1 << f;
+        cg.neu = neumann();
         cg.kz = cheb_kz;
         return cg;
     }
@@ -508,25 +517,29 @@ struct ChebStage : Stage {
             }
         }
     }
-    int apply(Field out, Field in, const int* gate) override
+    int apply(Field out, Field in, const int* gate) override { return run(out, in, gate, true); }
+    // the fused sweeps form every ghost themselves
+    int apply_internal(Field out, Field in, const int* gate) override
+    {
+        return run(out, in, gate, !(C.cheb_fused_ok() && cfg.max_iter >= 4));
+    }
+    int run(Field out, Field in, const int* gate, bool reset_ghosts)
     {
         int rc = buffers();
         if (rc) return rc;
         calls++;
         // resetNeumanBCs on the input (chebyshevIteration.hpp:74), in place
+        if (reset_ghosts) C.ghost(in, false, nullptr, gate);
         if (prec() == 64 && in.prec == 64) {
-            C.ghost(in, false, nullptr, gate);
             if (out.prec == 64) sweeps<double, double>(in.d(), out.d(), gate, Y, Z, W, V);
             else return C.fail(PPS_ERR_UNSUPPORTED, "FP64 Chebyshev into an FP32 field");
         } else {
             // CastPrecisionFieldKernel (kernelsAlpakaChebyshev.hpp:7-18) then FP32 sweeps
             const float* B = nullptr;
             if (in.prec == 64) {
-                C.ghost(in, false, nullptr, gate);
                 launch_cast<double, float>(C.gbox(32), C.stream, in.d(), Bc.f(), gate);
                 B = Bc.f();
             } else {
-                C.ghost(in, false, nullptr, gate);
                 B = in.f();
             }
             if (out.prec == 64) sweeps<float, double>(B, out.d(), gate, Y, Z, W, V);
@@ -573,7 +586,7 @@ struct KrylovStage : Stage {
             NoneStage none(C, pps_stage{}, level + 1);
             return none.apply(out, in, gate);
         }
-        return pre->apply(out, in, gate);
+        return pre->apply_internal(out, in, gate);
     }
     int pre_apply_dot(Field out, Field in, const int* gate, Field dot, int* nblocks)
     {
@@ -769,26 +782,23 @@ struct BiCGStage : KrylovStage {
         launch_copy<double>(g, C.stream, r.d(), p.d());
         launch_copy<double>(g, C.stream, r.d(), r0.d());
         const int* gate = &S->done;
+        const int mir = C.neumann();  // K1 and K3 form the ghosts of their input themselves
         auto body = [&]() -> int {
             if (pw) {
-                C.ghost(p, false, nullptr, gate);
-                launch_bicg_k1<double>(g, C.stream, C.rb, p.d(), c, AMp.d(), r0.d(), S);
+                launch_bicg_k1<double>(g, C.stream, C.rb, mir, p.d(), c, AMp.d(), r0.d(), S);
             } else {
                 int e = pre_apply(Mp, p, gate);
                 if (e) return e;
-                C.ghost(Mp, false, nullptr, gate);
-                launch_bicg_k1<double>(g, C.stream, C.rb, Mp.d(), 1.0, AMp.d(), r0.d(), S);
+                launch_bicg_k1<double>(g, C.stream, C.rb, mir, Mp.d(), 1.0, AMp.d(), r0.d(), S);
             }
             launch_bicg_k2<double>(g, C.stream, r.d(), AMp.d(), S);
             if (pw) {
-                C.ghost(r, false, nullptr, gate);
-                launch_bicg_k3<double>(g, C.stream, C.rb, r.d(), c, Az.d(), r.d(), S);
+                launch_bicg_k3<double>(g, C.stream, C.rb, mir, r.d(), c, Az.d(), r.d(), S);
                 launch_bicg_k45<double>(g, C.stream, C.rb, x.d(), p.d(), c, r.d(), c, r.d(), Az.d(), r0.d(), S, main);
             } else {
                 int e = pre_apply(z, r, gate);
                 if (e) return e;
-                C.ghost(z, false, nullptr, gate);
-                launch_bicg_k3<double>(g, C.stream, C.rb, z.d(), 1.0, Az.d(), r.d(), S);
+                launch_bicg_k3<double>(g, C.stream, C.rb, mir, z.d(), 1.0, Az.d(), r.d(), S);
                 launch_bicg_k45<double>(g, C.stream, C.rb, x.d(), Mp.d(), 1.0, z.d(), 1.0, r.d(), Az.d(), r0.d(), S, main);
             }
             launch_bicg_k6<double>(g, C.stream, p.d(), r.d(), AMp.d(), S);

@@ -309,7 +309,11 @@ __global__ __launch_bounds__(kSThreads) void k_stencil(Geo g, Op op, RedBuf rb)
         hv = true;
     }
     const bool hin = hv && hi <= g.hi0 && hj <= g.hi1;
-    const long long hbase = (long long)g.ox + hi + (long long)g.px * hj;
+    // where a point's input is read: itself, or the mirror point of a ghost (g.mir)
+    auto mx = [&](int v) { return (g.mir & 1) && v == g.lo0 - 1 ? v + 2 : (g.mir & 2) && v == g.hi0 ? v - 2 : v; };
+    auto my = [&](int v) { return (g.mir & 4) && v == g.lo1 - 1 ? v + 2 : (g.mir & 8) && v == g.hi1 ? v - 2 : v; };
+    auto mz = [&](int v) { return (g.mir & 16) && v == g.lo2 - 1 ? v + 2 : (g.mir & 32) && v == g.hi2 ? v - 2 : v; };
+    const long long hbase = (long long)g.ox + mx(hi) + (long long)g.px * my(hj);
     const T cx = (T)g.cx, cy = (T)g.cy, cz = (T)g.cz;
 
     using Raw = typename RawOf<Op, T>::type;
@@ -326,10 +330,10 @@ __global__ __launch_bounds__(kSThreads) void k_stencil(Geo g, Op op, RedBuf rb)
         const int j = jt + ly + q * kSTY;
         act[q] = (i < g.hi0) && (j < g.hi1);
         inb[q] = (i <= g.hi0) && (j <= g.hi1);
-        base[q] = (long long)g.ox + i + (long long)g.px * j;
-        vm[q] = inb[q] ? st_value<Op, T>(op, st_raw<Op, T>(op, base[q] + g.plane * (k0 - 1))) : T(0);
+        base[q] = (long long)g.ox + mx(i) + (long long)g.px * my(j);
+        vm[q] = inb[q] ? st_value<Op, T>(op, st_raw<Op, T>(op, base[q] + g.plane * mz(k0 - 1))) : T(0);
         rc[q] = inb[q] ? st_raw<Op, T>(op, base[q] + g.plane * k0) : Raw{};
-        r1[q] = inb[q] ? st_raw<Op, T>(op, base[q] + g.plane * (k0 + 1)) : Raw{};
+        r1[q] = inb[q] ? st_raw<Op, T>(op, base[q] + g.plane * mz(k0 + 1)) : Raw{};
         if (act[q]) oc[q] = st_ox<NT>(op, base[q] + g.plane * k0);
         vc[q] = inb[q] ? st_value<Op, T>(op, rc[q]) : T(0);
     }
@@ -346,7 +350,7 @@ __global__ __launch_bounds__(kSThreads) void k_stencil(Geo g, Op op, RedBuf rb)
         const bool more = k + 1 < k1;
 #pragma unroll
         for (int q = 0; q < kRY; ++q) {
-            if (inb[q] && more) r2[q] = st_raw<Op, T>(op, base[q] + g.plane * (k + 2));
+            if (inb[q] && more) r2[q] = st_raw<Op, T>(op, base[q] + g.plane * mz(k + 2));
             if (act[q] && more) on[q] = st_ox<NT>(op, base[q] + g.plane * (k + 1));
         }
         Raw h2{};
@@ -1527,7 +1531,7 @@ struct OpBiK1 : Gate {
 };
 
 template <typename T>
-void launch_bicg_k1(const Geo& g, hipStream_t s, RedBuf rb, const T* Mp, double amp, T* AMp, const T* r0, Scal* S)
+void launch_bicg_k1(const Geo& g0, hipStream_t s, RedBuf rb, int mir, const T* Mp, double amp, T* AMp, const T* r0, Scal* S)
 {
     OpBiK1<T> op;
     op.gate = &S->done;
@@ -1536,6 +1540,8 @@ void launch_bicg_k1(const Geo& g, hipStream_t s, RedBuf rb, const T* Mp, double 
     op.r0 = r0;
     op.S = S;
     op.amp = (T)amp;
+    Geo g = g0;
+    g.mir = mir;
     run_stencil<T, 1>(g, s, op, rb);
 }
 
@@ -1587,7 +1593,7 @@ struct OpBiK3 : Gate {
 };
 
 template <typename T>
-void launch_bicg_k3(const Geo& g, hipStream_t s, RedBuf rb, const T* z, double az, T* Az, const T* r, Scal* S)
+void launch_bicg_k3(const Geo& g0, hipStream_t s, RedBuf rb, int mir, const T* z, double az, T* Az, const T* r, Scal* S)
 {
     OpBiK3<T> op;
     op.gate = &S->done;
@@ -1596,6 +1602,8 @@ void launch_bicg_k3(const Geo& g, hipStream_t s, RedBuf rb, const T* z, double a
     op.r = r;
     op.S = S;
     op.az = (T)az;
+    Geo g = g0;
+    g.mir = mir;
     run_stencil<T, 2>(g, s, op, rb);
 }
 
@@ -2653,9 +2661,9 @@ void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, floa
     template void launch_cg_B<T>(const Geo&, hipStream_t, RedBuf, T*, const T*, Scal*, bool);                  \
     template void launch_cg_rz<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, Scal*);                 \
     template void launch_pointwise<T>(const Geo&, hipStream_t, const T*, T*, double, const int*);              \
-    template void launch_bicg_k1<T>(const Geo&, hipStream_t, RedBuf, const T*, double, T*, const T*, Scal*);   \
+    template void launch_bicg_k1<T>(const Geo&, hipStream_t, RedBuf, int, const T*, double, T*, const T*, Scal*);   \
     template void launch_bicg_k2<T>(const Geo&, hipStream_t, T*, const T*, const Scal*);                       \
-    template void launch_bicg_k3<T>(const Geo&, hipStream_t, RedBuf, const T*, double, T*, const T*, Scal*);   \
+    template void launch_bicg_k3<T>(const Geo&, hipStream_t, RedBuf, int, const T*, double, T*, const T*, Scal*);   \
     template void launch_bicg_k45<T>(const Geo&, hipStream_t, RedBuf, T*, const T*, double, const T*, double, T*, \
                                      const T*, const T*, Scal*, bool);                                         \
     template void launch_bicg_k6<T>(const Geo&, hipStream_t, T*, const T*, const T*, const Scal*);             \

@@ -101,6 +101,8 @@ struct Geo {
     int nblocks;
     int kz_st;          // z-chunk of stencil launches
     int nt;             // store field outputs non-temporally (working set beyond the caches)
+    int mir;            // stencils: bit f = the input's ghosts beyond face f (x- x+ y- y+ z- z+) are not
+                        // read from memory but from the data point two cells inward
     double cx, cy, cz;  // 1/ds^2 per direction
 };
 
@@ -202,12 +204,13 @@ template <typename T>
 void launch_pointwise(const Geo& gbox, hipStream_t s, const T* in, T* out, double c, const int* gate);
 
 // ---- BiCGSTAB (BiCGSTAB.hpp:131-292) ----
+// mir: Neumann faces of Mp (k1) and z (k3), whose ghosts need not be set (Geo::mir)
 template <typename T>
-void launch_bicg_k1(const Geo& g, hipStream_t s, RedBuf rb, const T* Mp, double amp, T* AMp, const T* r0, Scal* S);
+void launch_bicg_k1(const Geo& g, hipStream_t s, RedBuf rb, int mir, const T* Mp, double amp, T* AMp, const T* r0, Scal* S);
 template <typename T>
 void launch_bicg_k2(const Geo& g, hipStream_t s, T* r, const T* AMp, const Scal* S);
 template <typename T>
-void launch_bicg_k3(const Geo& g, hipStream_t s, RedBuf rb, const T* z, double az, T* Az, const T* r, Scal* S);
+void launch_bicg_k3(const Geo& g, hipStream_t s, RedBuf rb, int mir, const T* z, double az, T* Az, const T* r, Scal* S);
 template <typename T>
 void launch_bicg_k45(const Geo& g, hipStream_t s, RedBuf rb, T* x, const T* Mp, double amp, const T* z, double az,
                      T* r, const T* Az, const T* r0, Scal* S, bool history);
