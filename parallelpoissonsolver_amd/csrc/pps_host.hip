@@ -295,22 +295,26 @@ template <class Body>
 static int run_loop(Ctx& C, Scal* S, int maxit, bool host_each, Body body, int bodies_per_it = 1)
 {
     if (maxit <= 0) return PPS_OK;  // while (iter < maxIteration) never runs
-    // Batch size: 4 doubling, then sized from the measured time per iteration
-    // so that a batch holds about kBatchMs of device work (at most 64
-    // iterations).  Iterations queued past convergence retire as gated empty
-    // launches of a few microseconds each; with expensive iterations (the
-    // learned preconditioner: milliseconds) a 64-iteration batch would leave
-    // up to ~100 of them, with cheap ones (small grids) the host needs the
-    // large batches to stay ahead.
-    constexpr double kBatchMs = 5.0;
+    // Batch size: 4, then from the measured time per iteration.  Iterations
+    // queued past convergence retire as gated empty launches of 2-3 us each, up
+    // to two batches of them, and a batch boundary costs the device nothing as
+    // long as another batch is queued: so a batch holds a tenth of the loop's
+    // time so far, between 0.3 ms (what the host needs to stay ahead) and 5 ms,
+    // at most 64 iterations.  Against 4 doubling to 5 ms: the 10-iteration
+    // Chebyshev-preconditioned solve of 18^3 points 7.3 -> 4.4 ms (its outer
+    // corrections each end a loop).
+    auto batch_for = [](double ms_per_it, double elapsed_ms) {
+        const double target = std::max(0.3, std::min(5.0, 0.1 * elapsed_ms));
+        return std::max(1, std::min(64, (int)std::ceil(target / ms_per_it)));
+    };
     using clock = std::chrono::steady_clock;
     int batch = host_each ? 1 : 4;
     long long queued = 0;
     int slot = 0;
     bool have_prev = false;
     int n_slot[2] = {0, 0};  // iterations of the batch behind each event
-    clock::time_point t_done{};
-    bool have_done = false;
+    const clock::time_point t_begin = clock::now();
+    clock::time_point t_done = t_begin;
     for (;;) {
         const int nb = batch;
         for (int b = 0; b < nb; ++b) {
@@ -327,7 +331,6 @@ static int run_loop(Ctx& C, Scal* S, int maxit, bool host_each, Body body, int b
         rc = C.hip(hipGetLastError(), "kernel launch");
         if (rc) return rc;
         const int waitslot = host_each ? slot : slot ^ 1;
-        double ms_per_it = 0.0;
         if (host_each || have_prev) {
             rc = C.hip(hipEventSynchronize(C.ev_batch[waitslot]), "event sync");
             if (rc) return rc;
@@ -335,19 +338,13 @@ static int run_loop(Ctx& C, Scal* S, int maxit, bool host_each, Body body, int b
             // with two batches in flight the device ran the waited batch
             // between the two completions the host saw
             const clock::time_point now = clock::now();
-            if (have_done && n_slot[waitslot] > 0)
-                ms_per_it = std::chrono::duration<double, std::milli>(now - t_done).count() / n_slot[waitslot];
+            const double ms_per_it = std::chrono::duration<double, std::milli>(now - t_done).count() / n_slot[waitslot];
             t_done = now;
-            have_done = true;
+            if (!host_each)
+                batch = batch_for(ms_per_it, std::chrono::duration<double, std::milli>(now - t_begin).count());
         }
         have_prev = true;
         slot ^= 1;
-        if (!host_each) {
-            if (ms_per_it > 0.0)
-                batch = std::max(1, std::min(64, (int)std::ceil(kBatchMs / ms_per_it)));
-            else
-                batch = std::min(batch * 2, 64);
-        }
         if (queued > (long long)bodies_per_it * maxit + 2 * 64) break;  // every gate is closed by now
     }
     return C.hip(hipStreamSynchronize(C.stream), "sync");
