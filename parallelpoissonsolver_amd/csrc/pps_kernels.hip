@@ -1304,13 +1304,14 @@ struct OpCgPass {
         if (S->recheck) {
             // the pass formed r (x has its step already) and kept p
             S->recheck = 0;
-            S->v[S_BETA] = rr / S->v[S_RR];
+            S->v[S_BETA] = rr > 0.0 ? rr / S->v[S_RR] : 0.0;
             S->v[S_ALPHA] = 0.0;
             if (slot >= 0) S->ahist[slot] = 0.0;
             end_iteration(S->iter, rr);
             return;
         }
-        const double rz = S->v[S_JAC] * rr, a = rz / t[1];
+        // r = 0: x is exact and no step follows
+        const double rz = S->v[S_JAC] * rr, a = rr == 0.0 ? 0.0 : rz / t[1];
         S->v[S_RZ] = rz;
         S->v[S_PAP] = t[1];
         S->v[S_ALPHA] = a;

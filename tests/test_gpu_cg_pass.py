@@ -127,3 +127,22 @@ def test_one_pass_fp32_inner_cg(n):
     assert np.linalg.norm(b[sl] - apply_a(x, ds)) < 1.1e-12 * np.linalg.norm(b[sl])
     assert res["outer_iterations"] <= 6
     C.close()
+
+
+@pytest.mark.parametrize("deferred", [True, False])
+def test_iterations_past_an_exact_solution_stay_finite(deferred):
+    """tol = 0 on a grid whose residual underflows to zero before maxit."""
+    import parallelpoissonsolver_amd._lib as L
+    n = (6, 5, 4)
+    C, ds, sl = context(L, n, (0, 0, 0, 0, 0, 0))
+    C.set_deferred_x(deferred)
+    b = np.zeros(C.shape)
+    b[sl] = np.random.default_rng(3).normal(size=b[sl].shape)
+    C.fill(L.FIELD_X, 0.0)
+    C.upload(L.FIELD_B, b)
+    C.solve([dict(kind=L.IR, tol=1e-12, maxit=30),
+             dict(kind=L.CG, tol=0.0, maxit=400, precision=32), dict(kind=L.NONE)])
+    got = C.download(L.FIELD_X)[sl]
+    C.close()
+    r = b[sl] - apply_a(got, ds)
+    assert np.linalg.norm(r) <= 1e-10 * np.linalg.norm(b[sl])
