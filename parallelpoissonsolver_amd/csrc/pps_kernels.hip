@@ -1051,27 +1051,28 @@ __device__ __forceinline__ void ring_point(int t, int& r, int& c)
     else { r = t - 2 * (W + 2) - H; c = W; }
 }
 
-// z-chunk of a marching kernel whose blocks load `extra` planes beyond their
-// own and of which `slots` run at once: the one with the least work in the
-// busiest slot, ceil(blocks / slots) * (kz + extra) planes (the longest of
-// equals, up to 128 planes)
-static int pick_kz(long long tiles, int nz, int slots, int extra)
+constexpr int kCUs = 256;  // compute units of the MI355X
+
+// z-chunk of a marching kernel whose blocks take kz + extra steps and of which
+// per_cu (1 or 2) fit on a CU: the one with the least time on the busiest CU (the
+// longest of equals, up to 128 planes).  Two blocks that share a CU take 1.5 times
+// as long as one alone (Chebyshev(11), Dirichlet, us per BiCGSTAB iteration, chunk
+// of one / two blocks per CU: 98^3 200 / 215, 130^3 258 / 270).
+static int pick_kz(long long tiles, int nz, int per_cu, int extra)
 {
     int best = 1;
-    long long cost = -1;
+    double cost = -1.0;
     for (int kz = 1; kz <= 128; ++kz) {
         if (kz > 1 && kz > nz) break;
-        const long long nb = tiles * ((nz + kz - 1) / kz);
-        const long long c = ((nb + slots - 1) / slots) * (std::min(kz, nz) + extra);
-        if (cost < 0 || c <= cost) {
+        const long long n = (tiles * ((nz + kz - 1) / kz) + kCUs - 1) / kCUs;  // blocks of the busiest CU
+        const double c = (per_cu == 2 ? (n / 2) * 1.5 + n % 2 : (double)n) * (std::min(kz, nz) + extra);
+        if (cost < 0.0 || c <= cost) {
             cost = c;
             best = kz;
         }
     }
     return best;
 }
-
-constexpr int kCUs = 256;  // compute units of the MI355X
 
 // ------------------------------------------------------------------- CG
 
@@ -1349,8 +1350,8 @@ void launch_cg_pass(const Geo& g0, hipStream_t s, RedBuf rb, const T* r_in, cons
     const int nx = g0.hi0 - g0.lo0, ny = g0.hi1 - g0.lo1, nz = g0.hi2 - g0.lo2;
     if (nx <= 0 || ny <= 0 || nz <= 0) return;
     auto tiles = [&](int th) { return (long long)((nx + kTX - 1) / kTX) * ((ny + th - 1) / th); };
-    auto tiling = [&](int th, int slots) {
-        return retile(g0, th, g0.kz_st > 0 ? g0.kz_st : pick_kz(tiles(th), nz, slots, 4));
+    auto tiling = [&](int th, int per_cu) {
+        return retile(g0, th, g0.kz_st > 0 ? g0.kz_st : pick_kz(tiles(th), nz, per_cu, 4));
     };
     // 32-row tiles (one block per CU: 158 VGPRs) read fewer ring points and win
     // where there is enough work for two 16-plane chunks per CU, 16-row tiles (two
@@ -1358,8 +1359,8 @@ void launch_cg_pass(const Geo& g0, hipStream_t s, RedBuf rb, const T* r_in, cons
     // 1110 / 1169, 258^3 145 / 148, 194^3 77.5 / 71.5, 130^3 32.8 / 27.1, 66^3 15.5 / 13.9
     // (and where the last row of 32-row tiles is more than half full)
     const bool tall = tiles(4 * kCgW) * nz >= 2ll * 16 * kCUs && (ny - 1) % (4 * kCgW) + 1 > 2 * kCgW;
-    if (tall) run_cg_pass<T, 4>(tiling(4 * kCgW, kCUs), s, A, op, rb);
-    else run_cg_pass<T, 2>(tiling(2 * kCgW, 2 * kCUs), s, A, op, rb);
+    if (tall) run_cg_pass<T, 4>(tiling(4 * kCgW, 1), s, A, op, rb);
+    else run_cg_pass<T, 2>(tiling(2 * kCgW, 2), s, A, op, rb);
 }
 
 // buffer-preconditioned CG: p_new = z + beta*p_old, Ap = A p_new, p.Ap ; alpha = rz / pAp
@@ -1836,10 +1837,14 @@ void launch_cheb_sweep(const Geo& g, hipStream_t s, const T* Y, const T* B, cons
 // register.  A level's other points off the solver region are 0; B's, which the
 // first pass's start reads, are whatever the field holds there.
 //
-// Measured at 512^3 FP64: three sweeps in 1.30 ms (4.1 TB/s of its 5 words; 4.5
-// with the rings' re-reads that miss L2), 0.43 ms per sweep, where the pair took
-// 1.08 ms and needed a ghost fill per pass with Neumann faces.  The instruction
-// issue is a third of the time; the waves wait for memory and the barrier.
+// Measured at 512^3 FP64: three sweeps in 1.27 ms (4.2 TB/s of its 5 words; 4.6
+// with the rings' re-reads that miss L2), 0.42 ms per sweep, where the pair took
+// 1.08 ms and needed a ghost fill per pass with Neumann faces.  On grids that stay
+// in the caches the steps' instructions are half of the time, so plane pointers
+// are advanced instead of formed from the plane's number and two steps make a trip
+// of the loop, which makes the LDS planes constants: 2-5 % at every size (us per
+// BiCGSTAB + Chebyshev(24) iteration: 66^3 231 -> 226, mixed 130^3 756 -> 715,
+// 258^3 3000 -> 2905, 514^3 23450 -> 22920).
 constexpr int kChW = 8;   // wavefronts per block
 
 template <typename T, typename TO>
@@ -1962,8 +1967,20 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
         oc = buf_ld<T>(yb, ro[S - 1]);
     }
 
-    for (int s = s0; s <= s1; ++s) {
-        const int buf = s & 1, alt = buf ^ 1;
+    // plane k of a field with bound n: in [lo, lo + n) it is read or written
+    const long long pb = g.plane * (long long)sizeof(T);
+    const int ylo = first ? 0 : g.lo2, yend = min(first ? cg.ng[2] : g.hi2, s1 + 2);  // no step after s1 reads
+    const int zend = first ? g.lo2 : min(g.hi2, s1 + 1);                             // the first pass reads only Y
+    auto within = [](int k, int lo, int hi) { return (unsigned)(k - lo) < (unsigned)max(hi - lo, 0); };
+    const char *y2p = (const char*)(Yo + g.plane * (s0 + 2)), *z1p = (const char*)(Zo + g.plane * (s0 + 1)),
+               *b1p = (const char*)(Bo + g.plane * (s0 + 1));
+    char* wpp = (char*)((A.Wp ? A.Wp : (T*)A.Y) + org + g.plane * (s0 - (S - 2)));  // plane of level S - 1
+    char* wp = (char*)(A.W + org + g.plane * (s0 - (S - 1)));                       // plane of level S
+    const T c0 = first ? A.c0 : T(1);  // Z of the second sweep is c0 B on the first pass
+
+    // one step; BUF: the LDS planes that it writes, a constant so that the LDS addresses are
+    auto one = [&](const int s, auto BUF) __attribute__((always_inline)) {
+        const int buf = BUF, alt = buf ^ 1;
         // Y of plane s into LDS
 #pragma unroll
         for (int q = 0; q < RY; ++q) ysl[buf][jr + q + S][lx + S] = t[q].yc;
@@ -1973,10 +1990,10 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
         if (has[S - 1]) ysl[buf][pr[S - 1] + S][pc[S - 1] + S] = oc;
         // loads for the next step: Y of plane s + 2 (s + 1 on the outermost ring), Z and B of plane s + 1
         {
-            const auto y1 = plane_rsrc(Yo + g.plane * (s + 1), s < s1 && yin(s + 1));
-            const auto y2 = plane_rsrc(Yo + g.plane * (s + 2), s < s1 && yin(s + 2));
-            const auto z1 = plane_rsrc(Zo + g.plane * (s + 1), s < s1 && !first && zin(s + 1));
-            const auto b1 = plane_rsrc(Bo + g.plane * (s + 1), s < s1 && !first && zin(s + 1));
+            const auto y1 = plane_rsrc(y2p - pb, within(s + 1, ylo, yend));
+            const auto y2 = plane_rsrc(y2p, within(s + 2, ylo, yend));
+            const auto z1 = plane_rsrc(z1p, within(s + 1, g.lo2, zend));
+            const auto b1 = plane_rsrc(b1p, within(s + 1, g.lo2, zend));
             auto fetch = [&](ChebPoint<T>& P, unsigned o) {
                 P.yn = buf_ld<T>(y2, o);
                 P.zn = buf_ld<T>(z1, o);
@@ -2008,12 +2025,15 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
         // level 1 of plane s
         {
             const bool zs = zin(s);
-            auto level1 = [&](ChebPoint<T>& P, T Av) {
+            auto level1 = [&](ChebPoint<T>& P, T Av, bool in) {
+                T w;
                 if (first) {
                     P.bc = P.yc;
-                    return cheb_start(A.c1, A.c0, P.yc, Av);
+                    w = cheb_start(A.c1, A.c0, P.yc, Av);
+                } else {
+                    w = cheb_level(A.a[0], P.yc, A.b[0], P.bc, Av, A.c[0], P.zc);
                 }
-                return cheb_level(A.a[0], P.yc, A.b[0], P.bc, Av, A.c[0], P.zc);
+                P.un = in ? w : T(0);
             };
             auto at = [&](const ChebPoint<T>& P, int row, int col) {
                 const T(*y)[kTX + 2 * S] = ysl[buf];
@@ -2032,28 +2052,29 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
 #pragma unroll
                 for (int q = 0; q < RY; ++q) Av[q] = at(t[q], jr + q + dr[q] + S, lx + dc + S);
             }
-            const auto wr = plane_rsrc((A.Wp ? A.Wp : (T*)A.Y) + org + g.plane * s, S == 2 && A.Wp && s >= k0 && s < k1);
+            const auto wr = plane_rsrc(wpp, S == 2 && A.Wp && within(s, k0, k1));
 #pragma unroll
             for (int q = 0; q < RY; ++q) {
-                T w = level1(t[q], Av[q]);
-                if (!(val[q] && zs)) w = T(0);
-                t[q].un = w;
-                usl[buf][jr + q + S - 1][lx + S - 1] = w;
-                if constexpr (S == 2) buf_st<NT>(wr, so[q], w);
+                if (zs) level1(t[q], Av[q], val[q]);
+                else t[q].un = T(0);
+            }
+#pragma unroll
+            for (int q = 0; q < RY; ++q) {
+                usl[buf][jr + q + S - 1][lx + S - 1] = t[q].un;
+                if constexpr (S == 2) buf_st<NT>(wr, so[q], t[q].un);
             }
 #pragma unroll
             for (int d = 0; d < S - 1; ++d) {
                 if (!has[d]) continue;
-                T w = level1(r[d], at(r[d], mr[d] + S, mc[d] + S));
-                if (!(rv[d] && zs)) w = T(0);
-                r[d].un = w;
-                usl[buf][pr[d] + S - 1][pc[d] + S - 1] = w;
+                if (zs) level1(r[d], at(r[d], mr[d] + S, mc[d] + S), rv[d]);
+                else r[d].un = T(0);
+                usl[buf][pr[d] + S - 1][pc[d] + S - 1] = r[d].un;
             }
         }
         // level 2 of plane s - 1 (level 1 of that plane is in the other LDS buffer)
         if (s >= s0 + 2) {
             const int p = s - 1;
-            const bool zs = zin(p), own = p >= k0 && p < k1;
+            const bool zs = zin(p), own = within(p, k0, k1);
             if constexpr (NEU) {
                 const bool zlo = (cg.neu & 16) && p == cg.lo_d[2], zhi = (cg.neu & 32) && p == cg.hi_d[2] - 1;
                 auto mirror = [&](ChebPoint<T>& P) {
@@ -2067,7 +2088,7 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
                 }
             }
             auto level2 = [&](const ChebPoint<T>& P, T Av) {
-                return cheb_level(A.a[1], P.uc, A.b[1], P.b1, Av, A.c[1], first ? A.c0 * P.ym : P.ym);
+                return cheb_level(A.a[1], P.uc, A.b[1], P.b1, Av, A.c[1], c0 * P.ym);
             };
             auto at = [&](const ChebPoint<T>& P, int row, int col) {
                 const T(*u)[kTX + 2 * (S - 1)] = usl[alt];
@@ -2086,15 +2107,15 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
 #pragma unroll
                 for (int q = 0; q < RY; ++q) Av[q] = at(t[q], jr + q + dr[q] + S - 1, lx + dc + S - 1);
             }
-            const auto wr = plane_rsrc((A.Wp ? A.Wp : (T*)A.Y) + org + g.plane * p, S == 3 && A.Wp && own);
-            const auto xr = plane_rsrc(A.W + org + g.plane * p, S == 2 && own);
+            const auto wr = plane_rsrc((T*)wpp, S == 3 && A.Wp && own);
+            const auto xr = plane_rsrc((TO*)wp, S == 2 && own);
 #pragma unroll
             for (int q = 0; q < RY; ++q) {
                 T w = level2(t[q], Av[q]);
                 if constexpr (S == 2) {
                     buf_st<NT>(xr, so[q] == kOob ? kOob : so[q] * (unsigned)(sizeof(TO) / sizeof(T)), (TO)(A.sign * w));
                 } else {
-                    if (!(val[q] && zs)) w = T(0);
+                    w = val[q] && zs ? w : T(0);
                     t[q].vn = w;
                     vsl[alt][jr + q + 1][lx + 1] = w;
                     buf_st<NT>(wr, so[q], w);
@@ -2122,7 +2143,7 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
                         }
                     }
                 }
-                const auto xr = plane_rsrc(A.W + org + g.plane * p, true);
+                const auto xr = plane_rsrc((TO*)wp, true);
 #pragma unroll
                 for (int q = 0; q < RY; ++q) {
                     const int row = jr + q + 1, col = lx + 1;
@@ -2154,16 +2175,32 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
 #pragma unroll
         for (int d = 0; d < S - 1; ++d) step(r[d]);
         oc = on;
+        y2p += pb;
+        z1p += pb;
+        b1p += pb;
+        wpp += pb;
+        wp += g.plane * (long long)sizeof(TO);
+    };
+    if constexpr (sizeof(T) == 8 && S == 3 && RY == 2 && !NEU) {
+        // 128 registers, all in use: two steps per trip spill 15 (130^3 506 -> 586 us)
+        for (int s = s0; s <= s1; ++s) one(s, (s - s0) & 1);
+    } else {
+        for (int s = s0;;) {
+            one(s, std::integral_constant<int, 0>{});
+            if (++s > s1) break;
+            one(s, std::integral_constant<int, 1>{});
+            if (++s > s1) break;
+        }
     }
 }
 
 template <typename T, typename TO, int S, int RY>
-static void run_cheb_multi(const Geo& g0, const ChebPairGeo& cg, hipStream_t s, const ChebArgs<T, TO>& A, int slots)
+static void run_cheb_multi(const Geo& g0, const ChebPairGeo& cg, hipStream_t s, const ChebArgs<T, TO>& A, int per_cu)
 {
     constexpr int TY = kChW * RY;
     const int nx = g0.hi0 - g0.lo0, ny = g0.hi1 - g0.lo1, nz = g0.hi2 - g0.lo2;
     const long long tiles = (long long)((nx + kTX - 1) / kTX) * ((ny + TY - 1) / TY);
-    const Geo g = retile(g0, TY, cg.kz > 0 ? cg.kz : pick_kz(tiles, nz, slots, 2 * S));
+    const Geo g = retile(g0, TY, cg.kz > 0 ? cg.kz : pick_kz(tiles, nz, per_cu, 2 * S));
     const dim3 grid(g.nblocks), block(kTX, kChW);
     if (cg.neu && g.nt) hipLaunchKernelGGL((k_cheb_multi<T, TO, S, RY, true, true>), grid, block, 0, s, g, cg, A);
     else if (cg.neu) hipLaunchKernelGGL((k_cheb_multi<T, TO, S, RY, true, false>), grid, block, 0, s, g, cg, A);
@@ -2202,10 +2239,10 @@ void launch_cheb_multi(const Geo& g, const ChebPairGeo& cg, hipStream_t s, int s
     const int nx = g.hi0 - g.lo0, ny = g.hi1 - g.lo1, nz = g.hi2 - g.lo2, tail = (ny - 1) % (4 * kChW) + 1;
     const long long tiles = (long long)((nx + kTX - 1) / kTX) * ((ny + 4 * kChW - 1) / (4 * kChW));
     const bool tall = tiles * nz >= 8ll * kCUs && tail > 2 * kChW;
-    if (sweeps == 3 && tall) run_cheb_multi<T, TO, 3, 4>(g, cg, s, A, kCUs);
-    else if (sweeps == 3) run_cheb_multi<T, TO, 3, 2>(g, cg, s, A, cg.neu && sizeof(T) == 8 ? kCUs : 2 * kCUs);
-    else if (tall) run_cheb_multi<T, TO, 2, 4>(g, cg, s, A, kCUs);
-    else run_cheb_multi<T, TO, 2, 2>(g, cg, s, A, 2 * kCUs);
+    if (sweeps == 3 && tall) run_cheb_multi<T, TO, 3, 4>(g, cg, s, A, 1);
+    else if (sweeps == 3) run_cheb_multi<T, TO, 3, 2>(g, cg, s, A, cg.neu && sizeof(T) == 8 ? 1 : 2);
+    else if (tall) run_cheb_multi<T, TO, 2, 4>(g, cg, s, A, 1);
+    else run_cheb_multi<T, TO, 2, 2>(g, cg, s, A, 2);
 }
 
 // ------------------------------------------------------------------ FCG
