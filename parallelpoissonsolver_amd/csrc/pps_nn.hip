@@ -1246,104 +1246,118 @@ void launch_lift(const ConvArgs& a, hipStream_t s)
 // Inference form of the output layer with the lift fused in:
 //   z = out(up(E1) + relu(lift(r)))
 // so the 16-channel level-0 activation never goes to HBM.  A block owns a
-// 14 x 18 output tile; its X region (tile + 1-voxel halo) is 16 x 20 voxels,
-// one 16-voxel x-row per MFMA group, 5 rows per wavefront.  Per plane s and row:
+// 14 x 16 output tile, each wavefront 4 rows of it and the 6 x-rows of X (16
+// voxels, the tile with a 1-voxel halo) that they read.  Per plane s and x-row:
 //   1. lift: two K = 32 MFMAs over quad pairs of the input ring (64 slots
 //      for the 27 taps, the rest with zero weights; accumulator started at
-//      the bias, or at -1e30 outside the domain so that relu gives the zero
-//      padding); lane (voxel n, block j) then holds channels
+//      the bias, or at -1e30 outside the domain in x so that relu gives the
+//      zero padding); lane (voxel n, block j) then holds channels
 //      4j .. 4j+3; relu + BF16 in packed 16-bit form.  With e = up(E1) of the
-//      same channels, (a, e) is lane (n, j)'s A operand X;
-//   2. row partials P[dz,dy][n] = sum_dx sum_ci W[dz,dy,dx][ci] (a + e)[n+dx-1][ci]:
-//      X shifted one voxel left and right inside the 16-lane row (DPP), three
-//      MFMAs (one per dx) into columns m = 3 dz + dy; the skip sum a + e
-//      happens inside the MFMA (the weight operand repeats W[.][4j .. 4j+3]
-//      for both halves).  The 9 rows go to LDS as 16-byte writes of 4 voxels;
-// in the next step (after its one barrier) every thread adds the 9 partials of
-// its output voxel (rows y-1 .. y+1) into three running output planes; the
-// gather of plane s completes output plane s-1.
-// The output columns are 1 .. 14 of each row, so a shift never reaches past
-// the row for a value that is used.  With a.dot set the kernel also sums
-// z . dot over its outputs (FP64) and writes one partial per block to a.dpart
-// (the Krylov step's gamma = z . Ap_old without another pass over z).  The unfused path rounds a + e to BF16
-// before its MFMA; here the sum is exact, so outputs differ from it by that
-// rounding (relative ~1e-3 at most) and FP32 order.
-constexpr int kFW = 14, kFH = 18;                 // output tile
-constexpr int kXW = kFW + 2, kXH = kFH + 2;       // X region: 16 x 20
-constexpr int kFRW = kXW + 2, kFRH = kXH + 2;     // input ring plane: 18 x 22
+//      same channels, (a, e) is lane (n, j)'s B operand X; the skip sum a + e
+//      happens inside the next MFMAs (the weights repeat W[.][4j .. 4j+3] for
+//      both halves);
+//   2. three MFMAs (dy = 0, 1, 2) add the row into the accumulators of the three
+//      output rows it reaches.  Accumulator row 4 t + dx is the sum over dy, dz
+//      and the channels for output plane z with z mod 4 = t, kept across the
+//      planes s = z - 1 .. z + 1; the weight operand turns by one slot (4 lanes)
+//      per plane, read from LDS at the turned address, its fourth slot is zero.
+//      In C layout, lane (n, t) holds the three dx sums of voxel n.
+// Step s finishes output plane s - 2, whose slot is idle at plane s: the dx sums
+// meet by DPP inside the 16-lane row (columns 1 .. 14, so a shift never reaches
+// past the row for a value that is used), and three lane-block swaps bring the
+// wavefront's four rows, all in block t, to one row per block.  No partial goes
+// through LDS, which holds the input ring alone.  With a.dot set the kernel also
+// sums z . dot over its outputs (FP64) and writes one partial per block to a.dpart
+// (the Krylov step's gamma = z . Ap_old without another pass over z).  The unfused
+// path rounds a + e to BF16 before its MFMA; here the sum is exact, so outputs
+// differ from it by that rounding (relative ~1e-3 at most) and FP32 order.
+// Rows outside the domain are masked in the tiles that have any; the other tiles
+// run a copy of the march without masks.
+// Bound: issue and latency, not memory (2.1 GB a pass at 512^3).  A plane of a
+// wavefront is 24 MFMAs (384 cycles), about 75 vector instructions (300) and 14
+// LDS reads in about 820 cycles.  The form before it summed nine row partials per
+// voxel through LDS (9 reads, 40 DPP moves and 113 vector instructions per plane):
+// us per call with the gamma operand, 512^3 FP32 978 -> 880, 256^3 FP64 (gated
+// calls counted) 92 -> 84.  Occupancy decides: 3 blocks per CU 955 us; 5 blocks
+// spill in the plane loop (1440).  Weights turned by 12 DPP moves instead of the
+// LDS reads: 879.  14 x 16 and not wider: each further row costs an accumulator,
+// which 128 VGPRs do not have.
+constexpr int kFW = 14, kFR = 4;                  // output columns per tile, rows per wavefront
+constexpr int kFH = 4 * kFR;                      // output rows per tile
+constexpr int kXR = kFR + 2;                      // x-rows of X per wavefront
+constexpr int kFRW = kFW + 4, kFRH = kFH + 4;     // input ring plane: 18 x 20
 constexpr int kFRP = kFRW * kFRH;
-// quads per ring entry: the 396 positions, junk reads past the last row, and
+// quads per ring entry: the 360 positions, junk reads past the last row, and
 // the slots of the staging threads beyond the region (2 x 256), which store
 // their zeros there instead of branching
 constexpr int kQE = 512;
 static_assert(kQE >= kFRP + 4 && kQE >= 512, "ring entry holds the region, the junk reads and every staging slot");
-constexpr int kXQ = kXW * kXH;
-// P row stride: 4 mod 64 banks (measured: a stride of 8 mod 64 doubles the
-// bank conflicts of the 16-byte partial stores)
-constexpr int kXQp = kXQ + 4;
-constexpr int kFG = kXH / 4;                      // x-rows (groups) per wavefront
-static_assert(kXW == 16 && kXH % 4 == 0, "one 16-voxel x-row per group, equal rows per wavefront");
+static_assert(kFW + 2 == 16 && kFR == 4, "one 16-voxel x-row per MFMA, one output row per lane block");
 
-// (FP64 input: three blocks per CU, the raw FP64 prefetch does not fit the
-// register budget of four).  O64: the output field (and the dot operand) is
-// FP64; a template argument, so the plane loop holds one store and one
-// conversion.
+// a and b with a's upper (odd) blocks exchanged for b's lower (even) ones
+__device__ __forceinline__ void swap_halves(float& a, float& b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_blocks(float& a, float& b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+
+// O64: the output field (and the dot operand) is FP64; a template argument, so
+// the plane loop holds one store and one conversion.
 template <bool F64, bool O64>
 __global__ __launch_bounds__(256, 4) void k_outf(ConvArgs a, int zc)
 {
     if ((a.gate && *a.gate) || (a.gate2 && *a.gate2)) return;
     __shared__ __align__(16) u32x2 lq[2 * kQE];  // input quad ring: 2 entries
-    // P[3 dz + dy][voxel of the X region], double-buffered by X plane parity
-    // so that the partials of plane s and the gather of plane s - 1 share one
-    // barrier; the tail pads the gathers of the four threads without an
-    // output voxel
-    constexpr int kLPS = 9 * kXQp + 32;
-    __shared__ __align__(16) float lp[2 * kLPS];
     const int D = a.out.D, H = a.out.H, W = a.out.W;
     const TileIdx ti = tile_of_block();
     const int z0 = ti.z * zc;  // one sample
     const int z1 = min(z0 + zc, D);
     const int x0 = ti.x * kFW, y0 = ti.y * kFH;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane >> 4, n = lane & 15;
     // lift operands of the two quad-pair MFMAs
     const bf16x8 wqa = __builtin_bit_cast(bf16x8, ((const u32x4*)a.wl2)[lane]);
     const bf16x8 wqb = __builtin_bit_cast(bf16x8, ((const u32x4*)a.wl2)[64 + lane]);
-    bf16x8 wp[3];  // per dx: column m = 3 dz + dy
-#pragma unroll
-    for (int dx = 0; dx < 3; ++dx) wp[dx] = __builtin_bit_cast(bf16x8, ((const u32x4*)a.wl)[64 * dx + lane]);
+    // output weights per dy: row 4 t + dx, packed for planes 0 mod 4 (the first
+    // step's barrier stands before their first read)
+    __shared__ __align__(16) u32x4 lw[3 * 64];
+    if (tid < 3 * 64) lw[tid] = ((const u32x4*)a.wl)[tid];
     const float bout = a.bias ? a.bias[0] : 0.0f;
-    // X voxel of lane n: column gx; rows y0 - 1 + wave + 4k (k < kFG)
-    const int gx = x0 - 1 + n;
+    // X voxel of lane n: column gx; rows y0 - 1 + 4 wave + k (k < kXR)
+    const int gx = x0 - 1 + n, gy0 = y0 - 1 + kFR * wave;
     const bool xin = gx >= 0 && gx < W;
     unsigned yin = 0u;  // rows of this wavefront inside the domain
 #pragma unroll
-    for (int k = 0; k < kFG; ++k) {
-        const int gy = y0 - 1 + wave + 4 * k;
-        if (gy >= 0 && gy < H) yin |= 1u << k;
-    }
-    yin = __builtin_amdgcn_readfirstlane(yin);
+    for (int k = 0; k < kXR; ++k)
+        if (gy0 + k >= 0 && gy0 + k < H) yin |= 1u << k;
     // lift accumulators start at the bias, or at -1e30 outside the domain
     // (relu then gives the zero padding)
-    f32x4 cinit[kFG];
+    f32x4 cinit;
 #pragma unroll
-    for (int k = 0; k < kFG; ++k)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            cinit[k][r] = (xin && ((yin >> k) & 1u)) ? (a.bias2 ? a.bias2[4 * j + r] : 0.0f) : -1e30f;
-    // coarse activation E1: byte offset of this lane's 4 channels in row k
-    // (kOOB outside the domain: the load returns zeros)
+    for (int r = 0; r < 4; ++r) cinit[r] = xin ? (a.bias2 ? a.bias2[4 * j + r] : 0.0f) : -1e30f;
+    // coarse activation E1: byte offset of this lane's 4 channels in the coarse
+    // rows of X rows 0, 1-2, 3-4, 5 (kOOB outside: the load returns zeros)
+    constexpr int kER = kXR / 2 + 1;
     const int cW = a.in.W, cH = a.in.H;
     const long long cplane = (long long)cH * cW * kC;
-    const int cy0 = (y0 - 1 + wave) >> 1;  // coarse row of k = 0 (rows k step by 2)
-    unsigned eoff[kFG];
+    unsigned eoff[kER];
 #pragma unroll
-    for (int k = 0; k < kFG; ++k)
-        eoff[k] = (xin && ((yin >> k) & 1u)) ? (unsigned)(2 * (((cy0 + 2 * k) * cW + (gx >> 1)) * kC + 4 * j)) : kOOB;
-    // lift operand quads of this lane for X voxel (row wave, column n)
-    const int pa = (kQuad[0][j][0] + wave) * kFRW + kQuad[0][j][1] + n;
-    const int pb = (kQuad[1][j][0] + wave) * kFRW + kQuad[1][j][1] + n;
-    // input ring over the region (x0 - 2 .., y0 - 2 ..), 18 x 22 positions:
+    for (int k = 0; k < kER; ++k) {
+        const int cy = (gy0 >> 1) + k;
+        eoff[k] = (xin && cy >= 0 && cy < cH) ? (unsigned)(2 * ((cy * cW + (gx >> 1)) * kC + 4 * j)) : kOOB;
+    }
+    // lift operand quads of this lane for X voxel (row 4 wave, column n)
+    const int pa = (kQuad[0][j][0] + kFR * wave) * kFRW + kQuad[0][j][1] + n;
+    const int pb = (kQuad[1][j][0] + kFR * wave) * kFRW + kQuad[1][j][1] + n;
+    // input ring over the region (x0 - 2 .., y0 - 2 ..), 18 x 20 positions:
     // entry q mod 2 holds the quads (plane q-1, q, q+1, 0) of X plane q.  Each
     // staging thread keeps its slots' last two planes (BF16) in a register and
     // writes the whole quad of entry p-1 once plane p arrives.
@@ -1367,79 +1381,93 @@ __global__ __launch_bounds__(256, 4) void k_outf(ConvArgs a, int zc)
     };
     // up(E1) of this wavefront's rows, loaded one plane ahead (zeros outside
     // the domain)
-    u32x2 ev[kFG];
+    u32x2 ev[kER];
 #pragma unroll
-    for (int k = 0; k < kFG; ++k) ev[k] = u32x2{0u, 0u};
-    auto fetch_e = [&](u32x2* e, int s) {
+    for (int k = 0; k < kER; ++k) ev[k] = u32x2{0u, 0u};
+    auto fetch_e = [&](int s) {
         const __amdgpu_buffer_rsrc_t r = buf_rsrc(a.in.p + (s >> 1) * cplane, kInRange);
 #pragma unroll
-        for (int k = 0; k < kFG; ++k) e[k] = __builtin_amdgcn_raw_buffer_load_b64(r, eoff[k], 0, 0);
+        for (int k = 0; k < kER; ++k) ev[k] = __builtin_amdgcn_raw_buffer_load_b64(r, eoff[k], 0, 0);
     };
     // row k of X from the quad ring: lift (two MFMAs, relu to BF16) beside
-    // up(E1) as the partials' operand
-    auto lift_row = [&](const u32x2* q, const u32x2* e, int k) {
-        const u32x2 qa0 = q[pa + 4 * k * kFRW], qa1 = q[pa + 4 * k * kFRW + 1];
-        const u32x2 qb0 = q[pb + 4 * k * kFRW], qb1 = q[pb + 4 * k * kFRW + 1];
+    // up(E1); rows outside the domain are zero (EDGE: there may be some)
+    auto lift_row = [&](const u32x2* q, int k, auto edge_c) {
+        const u32x2 qa0 = q[pa + k * kFRW], qa1 = q[pa + k * kFRW + 1];
+        const u32x2 qb0 = q[pb + k * kFRW], qb1 = q[pb + k * kFRW + 1];
         const u32x4 ba = {qa0[0], qa0[1], qa1[0], qa1[1]}, bb = {qb0[0], qb0[1], qb1[0], qb1[1]};
-        f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wqa, __builtin_bit_cast(bf16x8, ba), cinit[k], 0, 0, 0);
+        f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wqa, __builtin_bit_cast(bf16x8, ba), cinit, 0, 0, 0);
         c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wqb, __builtin_bit_cast(bf16x8, bb), c, 0, 0, 0);
         u32x4 bx;
         bx[0] = relu_bf2(pack2bf(c[0], c[1]));
         bx[1] = relu_bf2(pack2bf(c[2], c[3]));
-        bx[2] = e[k][0];
-        bx[3] = e[k][1];
+        bx[2] = ev[(k + 1) / 2][0];
+        bx[3] = ev[(k + 1) / 2][1];
+        if constexpr (decltype(edge_c)::value) {
+            const unsigned m = ((yin >> k) & 1u) ? ~0u : 0u;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bx[r] &= m;
+        }
         return bx;
     };
-    // one plane of X -> tap partials, this wavefront's rows.  On FP32 fields
-    // the lift of row k + 1 is issued before the partials of row k so that
-    // the two chains overlap; the FP64 variant has no registers to spare for
-    // that at 4 blocks per CU.
-    auto partials = [&](const u32x2* e, int es) {
+    f32x4 acc[kFR];
+#pragma unroll
+    for (int i = 0; i < kFR; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // one plane of X into the accumulators.  The lift of row k + 1 is issued
+    // before row k's MFMAs so that the two chains overlap.
+    auto plane = [&](int s, int es, auto edge_c) {
         const u32x2* const q = lq + es * kQE;  // entry of X plane s (es = s mod 2)
-        u32x4 bx = lift_row(q, e, 0);
+        u32x4 wp[3];
+        const u32x4* const pw = lw + 16 * j + ((n - 4 * s) & 15);
 #pragma unroll
-        for (int k = 0; k < kFG; ++k) {
+        for (int dy = 0; dy < 3; ++dy) wp[dy] = pw[64 * dy];
+        u32x4 bx = lift_row(q, 0, edge_c);
+#pragma unroll
+        for (int k = 0; k < kXR; ++k) {
             u32x4 bn;
-            if (!F64 && k + 1 < kFG) bn = lift_row(q, e, k + 1);
-            // the row's neighbours: voxel n-1 (row_shr:1) and n+1 (row_shl:1)
-            u32x4 bm, bp;
+            if (k + 1 < kXR) bn = lift_row(q, k + 1, edge_c);
 #pragma unroll
-            for (int e8 = 0; e8 < 4; ++e8) {
-                bm[e8] = (unsigned)__builtin_amdgcn_mov_dpp((int)bx[e8], 0x111, 0xF, 0xF, true);
-                bp[e8] = (unsigned)__builtin_amdgcn_mov_dpp((int)bx[e8], 0x101, 0xF, 0xF, true);
-            }
-            f32x4 pr = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bm), wp[0],
-                                                               f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            pr = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bx), wp[1], pr, 0, 0, 0);
-            pr = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bp), wp[2], pr, 0, 0, 0);
-            // lane (column m, j): voxels 4j .. 4j+3 of row wave + 4k; the MFMA
-            // columns m >= 9 carry no partial
-            if (n < 9) *(f32x4*)(lp + es * kLPS + n * kXQp + (wave + 4 * k) * kXW + 4 * j) = pr;
-            if (k + 1 < kFG) bx = F64 ? lift_row(q, e, k + 1) : bn;
+            for (int dy = 0; dy < 3; ++dy)
+                if (k - dy >= 0 && k - dy < kFR)
+                    acc[k - dy] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, wp[dy]), __builtin_bit_cast(bf16x8, bx), acc[k - dy], 0, 0, 0);
+            if (k + 1 < kXR) bx = bn;
         }
     };
-    // this thread's output voxel: byte offset inside an output plane, kOOB
-    // for threads without one (their stores are dropped, dot loads give 0)
-    const int oy = tid / kFW, ox = tid - oy * kFW;
-    const int x = x0 + ox, y = y0 + oy;
-    const bool mine = tid < kFW * kFH && x < W && y < H;
-    const int q0 = oy * kXW + ox + 1;  // X region voxel of the output's (x, y - 1) neighbour
-    float am1 = 0.0f, a0 = 0.0f, ap1 = 0.0f;
+    // the finished sums of slot t: lane (n, j) gets voxel n of row j
+    auto finished = [&](int t) {
+        float v[kFR];
+#pragma unroll
+        for (int i = 0; i < kFR; ++i) {
+            // voxel n-1 (row_shr:1) at dx = 0 and n+1 (row_shl:1) at dx = 2
+            const float lo = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[i][0]), 0x111, 0xF, 0xF, true));
+            const float hi = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[i][2]), 0x101, 0xF, 0xF, true));
+            v[i] = (acc[i][1] + lo) + hi;
+        }
+        swap_halves(v[0], v[2]);  // blocks 0, 1 of both rows | blocks 2, 3
+        swap_halves(v[1], v[3]);
+        float p = (t & 2) ? v[2] : v[0], q = (t & 2) ? v[3] : v[1];
+        swap_blocks(p, q);
+        return (t & 1) ? q : p;
+    };
+    // this lane's output voxel: byte offset inside an output plane, kOOB
+    // for lanes without one (their stores are dropped, dot loads give 0)
+    const int y = y0 + kFR * wave + j;
+    const bool mine = n >= 1 && n <= kFW && gx < W && y < H;
     constexpr bool o64 = O64;
     constexpr int oesz = o64 ? 8 : 4;
-    const unsigned ooff = mine ? (unsigned)((x * a.fout.sx + y * a.fout.sy) * oesz) : kOOB;
+    const unsigned ooff = mine ? (unsigned)((gx * a.fout.sx + y * a.fout.sy) * oesz) : kOOB;
     const char* obase = (const char*)a.fout.p + a.fout.off * oesz;
     const char* dbase = a.dot ? (const char*)a.dot + a.fout.off * oesz : nullptr;
     const long long oszb = a.fout.sz * oesz;
     // dot operands: loaded with the input prefetch two steps ahead of their
     // output plane's step (one buffer per step parity, like the prefetch:
-    // step s loads the operand of output plane s) and converted where the step
-    // waits for that prefetch anyway.  The load is one 8-byte load in every
-    // case (an FP32 operand is its low word; a plane outside the chunk, or no
-    // dot at all, gets num_records 0): a load under a branch would make the
-    // compiler wait for the prefetch right after it.
-    u32x2 dA = {0u, 0u}, dB = {0u, 0u};
-    double dcur = 0.0, dacc = 0.0;
+    // step s loads the operand of output plane s) and used where the step
+    // waits for that prefetch anyway.  The load is unconditional (a plane
+    // outside the chunk, or no dot at all, gets num_records 0): a load under a
+    // branch would make the compiler wait for the prefetch right after it.
+    using Dot = std::conditional_t<O64, u32x2, unsigned>;
+    Dot dA{}, dB{}, dcur{};
+    double dacc = 0.0;
 
     // planes s = z0-1 .. z1 of X; the ring holds input planes s-1 .. s+1
     // planes z0 - 2 and z0 - 1 fill the slots' history (their quads land in
@@ -1450,63 +1478,50 @@ __global__ __launch_bounds__(256, 4) void k_outf(ConvArgs a, int zc)
     store_plane(preA, z0 - 1);
     fs.fetch(preA, z0, D);
     fs.fetch(preB, z0 + 1, D);
-    if (z0 >= 1) fetch_e(ev, z0 - 1);  // uniform
-    // step s: stage input plane s+1, partials of X plane s, gather of X plane
-    // s - 1 and output plane s - 2.  Two planes of input loads in flight,
-    // each buffer refilled once written; es = s mod 2: the ring entry and the
-    // partials buffer of X plane s.  One barrier per step: the ring entry of
-    // plane s is staged; the partials of plane s - 1 are complete; the gather
-    // of plane s - 2, which read the buffer that plane s fills, is done.
-    auto step = [&](int s, int es, Raw* buf, u32x2& dbuf, auto full_c, auto keep_c) {
+    if (z0 >= 1) fetch_e(z0 - 1);  // uniform
+    // step s: stage input plane s+1, output plane s - 2, X plane s into the
+    // accumulators.  Two planes of input loads in flight, each buffer refilled
+    // once written; es = s mod 2: the ring entry of X plane s.  One barrier per
+    // step: the ring entry of plane s is staged, and the reads of the other
+    // entry, which the next step rewrites, are done.
+    auto step = [&](int s, int es, Raw* buf, Dot& dbuf, auto full_c, auto keep_c, auto edge_c) {
         // FULL: a step of the chunk's interior (z0 + 2 <= s <= z1 - 2), which
         // has every part below; KEEP: s is even, so ev already holds the
         // coarse plane (s + 1) / 2 (loaded by step s - 1)
         constexpr bool FULL = decltype(full_c)::value, KEEP = decltype(keep_c)::value;
         store_plane(buf, s + 1);
-        {
-            const double d64 = __builtin_bit_cast(double, dbuf), d32 = (double)__uint_as_float(dbuf[0]);
-            if constexpr (O64) dcur = d64;  // the operand of output plane s-2
-            else dcur = d32;
-        }
+        dcur = dbuf;  // the operand of output plane s-2
         fs.fetch(buf, s + 3, D);  // zeros beyond the domain; unused beyond the chunk
         {
             const bool din = dbase != nullptr && s >= z0 && s < z1;  // uniform: output plane s
             const __amdgpu_buffer_rsrc_t r = buf_rsrc(din ? dbase + s * oszb : obase, din ? kInRange : 0);
-            dbuf = __builtin_amdgcn_raw_buffer_load_b64(r, ooff, 0, 0);
+            if constexpr (O64) dbuf = __builtin_amdgcn_raw_buffer_load_b64(r, ooff, 0, 0);
+            else dbuf = __builtin_amdgcn_raw_buffer_load_b32(r, ooff, 0, 0);
         }
         __syncthreads();
-        if (FULL || (s >= 0 && s < D && s <= z1)) partials(ev, es);  // uniform
-        if constexpr (!KEEP)
-            if (FULL || (s + 1 <= z1 && s + 1 < D)) fetch_e(ev, s + 1);
-        const int sg = s - 1;                        // X plane gathered
-        if (FULL || (sg >= 0 && sg < D && sg >= z0 - 1)) {  // uniform; every thread gathers,
-            const float* const lg = lp + (es ^ 1) * kLPS;  // those without an output read the padding
-            float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-            for (int dy = 0; dy < 3; ++dy) {
-                const float* pq = lg + dy * kXQp + q0 + dy * kXW;
-                s0 += pq[0];
-                s1 += pq[3 * kXQp];
-                s2 += pq[6 * kXQp];
-            }
-            am1 += s2;
-            a0 += s1;
-            ap1 += s0;
-        }
         const int zo = s - 2;
         if (FULL || (zo >= z0 && zo < z1)) {  // uniform
-            const float v = am1 + bout;
+            const float v = finished(zo & 3) + bout;
             const __amdgpu_buffer_rsrc_t r = buf_rsrc(obase + zo * oszb, kInRange);
             if constexpr (O64) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, (double)v), r, ooff, 0, 0);
             else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, ooff, 0, 0);
-            // threads without an output hold a dot operand of 0 but may hold a
-            // non-finite v (gathered from the padding)
-            const double pr = (double)v * dcur;
-            dacc += mine ? pr : 0.0;
+            // lanes without an output hold a dot operand of 0 but may hold a
+            // non-finite v
+            double dv;
+            if constexpr (O64) dv = __builtin_bit_cast(double, dcur);
+            else dv = (double)__uint_as_float(dcur);
+            dacc = fma((double)(mine ? v : 0.0f), dv, dacc);
         }
-        am1 = a0;
-        a0 = ap1;
-        ap1 = 0.0f;
+        // output plane s + 1 starts at plane s: its slot is cleared here and not
+        // when it is read, so that a non-finite X of the idle plane stays out
+        const bool fresh = j == ((s + 1) & 3);
+#pragma unroll
+        for (int i = 0; i < kFR; ++i)
+#pragma unroll
+            for (int r = 0; r < 3; ++r) acc[i][r] = fresh ? 0.0f : acc[i][r];
+        if (FULL || (s >= 0 && s < D && s <= z1)) plane(s, es, edge_c);  // uniform
+        if constexpr (!KEEP)
+            if (FULL || (s + 1 <= z1 && s + 1 < D)) fetch_e(s + 1);
     };
     // steps s = z0 - 1 .. z1 + 1 alternate the buffers A, B from A.  The
     // interior pairs run without a conditional step or part (a skipped step
@@ -1516,19 +1531,24 @@ __global__ __launch_bounds__(256, 4) void k_outf(ConvArgs a, int zc)
     // (chunks start on even planes, so the interior pairs start on even s)
     using T_ = std::true_type;
     using F_ = std::false_type;
-    step(z0 - 1, (z0 - 1) & 1, preA, dA, F_{}, F_{});
-    step(z0, z0 & 1, preB, dB, F_{}, F_{});
-    step(z0 + 1, (z0 + 1) & 1, preA, dA, F_{}, F_{});
-    int s = z0 + 2;
-    for (; s + 1 <= z1 - 2; s += 2) {
-        step(s, s & 1, preB, dB, T_{}, T_{});
-        step(s + 1, (s + 1) & 1, preA, dA, T_{}, F_{});
-    }
-    // the steps left up to z1 + 1: 3 or 4, or 1 or 2 for a chunk of 1 or 2 planes
-    if (s <= z1 + 1) step(s, s & 1, preB, dB, F_{}, F_{});
-    if (s + 1 <= z1 + 1) step(s + 1, (s + 1) & 1, preA, dA, F_{}, F_{});
-    if (s + 2 <= z1 + 1) step(s + 2, (s + 2) & 1, preB, dB, F_{}, F_{});
-    if (s + 3 <= z1 + 1) step(s + 3, (s + 3) & 1, preA, dA, F_{}, F_{});
+    auto march = [&](auto edge) {
+        step(z0 - 1, (z0 - 1) & 1, preA, dA, F_{}, F_{}, edge);
+        step(z0, z0 & 1, preB, dB, F_{}, F_{}, edge);
+        step(z0 + 1, (z0 + 1) & 1, preA, dA, F_{}, F_{}, edge);
+        int s = z0 + 2;
+        for (; s + 1 <= z1 - 2; s += 2) {
+            step(s, s & 1, preB, dB, T_{}, T_{}, edge);
+            step(s + 1, (s + 1) & 1, preA, dA, T_{}, F_{}, edge);
+        }
+        // the steps left up to z1 + 1: 3 or 4, or 1 or 2 for a chunk of 1 or 2 planes
+#pragma unroll 1
+        for (; s <= z1 + 1; s += 2) {
+            step(s, s & 1, preB, dB, F_{}, F_{}, edge);
+            if (s + 1 <= z1 + 1) step(s + 1, (s + 1) & 1, preA, dA, F_{}, F_{}, edge);
+        }
+    };
+    if (y0 >= 1 && y0 + kFH < H) march(F_{});  // every X row inside the domain
+    else march(T_{});
     if (a.dot) {
         __shared__ double red[4];
 #pragma unroll
@@ -1540,7 +1560,7 @@ __global__ __launch_bounds__(256, 4) void k_outf(ConvArgs a, int zc)
     }
 }
 
-// grid of the fused output kernel: 14 x 18 tiles, four resident blocks per CU
+// grid of the fused output kernel: 14 x 16 tiles, four resident blocks per CU
 static dim3 outf_grid(int D, int H, int W, int* zc)
 {
     const int tx = (W + kFW - 1) / kFW, ty = (H + kFH - 1) / kFH;
@@ -1940,8 +1960,9 @@ void launch_up_back(const ActRef& dx, const ActRef& dcoarse, hipStream_t s)
 // lift kernel: k = 4*(lane/16) + d holds plane d of the quad at dx = lane/16;
 // and from kLiftPairOff two K = 32 operands o for the fused output kernel:
 // k = 8*(lane/16) + e holds plane e%4 of quad e/4 of the pair kQuad[o][lane/16]
-// row partials (mode 3, 1 output channel): three operands o = dx, column
-// m = 3 dz + dy, k = 8*(lane/16) + e -> input channel 4*(lane/16) + e%4
+// output layer (mode 3, 1 output channel): three operands o = dy, row m = 4 t + dx
+// with dz = 1, 0, none, 2 for slot t, k = 8*(lane/16) + e -> input channel
+// 4*(lane/16) + e%4
 __global__ void k_pack(const float* __restrict__ W, int cin, int cout, int mode, uint16_t* __restrict__ wl)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1968,13 +1989,13 @@ __global__ void k_pack(const float* __restrict__ W, int cin, int cout, int mode,
             return;
         }
     } else if (mode == 3) {
-        // the fused output layer's row-partial weights: operand o = dx, column
-        // m = 3 dz + dy (m < 9), k = 8*(lane/16) + e -> input channel
-        // 4*(lane/16) + e%4 (the lift half and the skip half of the A operand
-        // share the weights)
+        // the fused output layer's weights for planes s = 0 mod 4: slot t holds
+        // output plane s (t = 0), s + 1 (1) or s - 1 (3); the lift half and the
+        // skip half of X share the weights
         if (t >= 3 * 512) return;
-        const int ci = 4 * j + (e & 3);
-        if (m < 9 && ci < cin && cout > 0) v = W[(9 * (m / 3) + 3 * (m % 3) + o) * 256 + ci * 16];
+        const int ci = 4 * j + (e & 3), slot = m >> 2, dx = m & 3;
+        const int dz = slot == 0 ? 1 : slot == 1 ? 0 : 2;
+        if (slot != 2 && dx < 3 && ci < cin && cout > 0) v = W[(9 * dz + 3 * o + dx) * 256 + ci * 16];
     } else {
         if (t >= kPackedHalves) return;
         const int p = o / 3, dy = o % 3, c = pair_combo(p, j >> 1), k = 8 * (j & 1) + e;
@@ -2171,7 +2192,7 @@ void Net::pack_all()
         hipLaunchKernelGGL(k_pack, dim3(kPackedHalves / 256), dim3(256), 0, stream_, W, kNet[l].cin, kNet[l].cout, 1,
                            wlt_ + (size_t)l * kPackedHalves);
     }
-    // the output layer again as row-partial operands, for the fused inference kernel
+    // the output layer again, laid out for the fused inference kernel
     hipLaunchKernelGGL(k_pack, dim3(6), dim3(256), 0, stream_, params_ + (size_t)(kLayers - 1) * kLayerParams,
                        kNet[kLayers - 1].cin, kNet[kLayers - 1].cout, 3, wlo_);
 }
