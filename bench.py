@@ -177,13 +177,15 @@ def host_cpu():
 def cpu_baseline(gpu_iterations):
     """Reference CPU solver (compiled from the reference sources into oracle/_ref)
     on the host cores: 100 CG iterations of the same 512^3 workload under MPI,
-    extrapolated to the iteration count the solve needs.  Fails loudly when the
-    reference build or mpirun is missing (pass --no-cpu to skip the baseline)."""
+    extrapolated to the iteration count the solve needs.  None, with a line in the
+    log, where the reference build or mpirun is missing (pass --no-cpu to skip the
+    baseline)."""
     exe = os.path.join(ROOT, "oracle", "_ref", "ref_solver_sample")
     mpirun = shutil.which("mpirun") or "/opt/conda/bin/mpirun"
     if not (os.path.exists(exe) and os.path.exists(mpirun)):
-        raise RuntimeError(f"CPU baseline: {exe} or mpirun missing (build with __graft_entry__.build() where the "
-                           f"reference sources are present, or pass --no-cpu)")
+        log(f"CPU baseline: not measured, {exe} or mpirun missing (build with __graft_entry__.build() where the "
+            f"reference sources are present)")
+        return None
     npg = N_INTERIOR + 2
     ds = 1.0 / (npg - 1)
     ranks = (2, 2, 2)  # 514 = 2 * 257: the reference needs ranks dividing npglobal (blockGrid.hpp:165)
