@@ -1558,8 +1558,8 @@ int pps_create(const pps_grid* grid, void** out)
     const long long nvec = (long long)((X.ng[0] + kThreads - 1) / kThreads) * X.ng[1] * X.ng[2];
     // one-plane chunks of 64 x 16 tiles (small grids' CG pass)
     const long long nsmall = (long long)((X.ng[0] + kTX - 1) / kTX) * ((X.ng[1] + 15) / 16) * X.ng[2];
-    // the network's output kernel: 14 x 18 tiles in chunks of 2 planes at least
-    const long long nout = (long long)((X.ng[0] + 13) / 14) * ((X.ng[1] + 17) / 18) * ((X.ng[2] + 1) / 2);
+    // the network's output kernel: 14 x 16 tiles in chunks of 2 planes at least
+    const long long nout = (long long)((X.ng[0] + 13) / 14) * ((X.ng[1] + 15) / 16) * ((X.ng[2] + 1) / 2);
     X.rb.cap = (int)std::max(std::max<long long>(gbig.nblocks, nvec), std::max(nsmall, nout)) + 8;
     X.rb.cap2 = X.rb.cap / kSpan + 8;
     rc = rc ? rc : X.hip(hipMalloc(&X.rb.partials2, sizeof(double) * kMaxRedQ * X.rb.cap2), "span partials");
