@@ -69,23 +69,17 @@ struct Stage {
     // apply() for a caller that does not read `in`'s Neumann ghosts afterwards:
     // they need not be reset in place
     virtual int apply_internal(Field out, Field in, const int* gate) { return apply(out, in, gate); }
-    // apply() that may also sum out . dot into the context's reduction
-    // partials: *nblocks = their count, or 0 when the stage does not
-    virtual int apply_dot(Field out, Field in, const int* gate, Field dot, int* nblocks)
-    {
-        (void)dot;
-        *nblocks = 0;
-        return apply(out, in, gate);
-    }
     // whether apply_update() is available: the stage forms its input as the
     // updated residual in = r_prev - alpha ap_prev (r_prev while *skip) and
-    // writes it to `in`, so the Krylov loop needs no update pass of its own
+    // writes it to `in`, so the Krylov loop needs no update pass of its own.  It may
+    // also sum out . dot into the context's reduction partials: nblocks[0] = their
+    // count, or 0 when it does not, nblocks[1] = their count while the fallback is on
     virtual bool forms_update() const { return false; }
     virtual int apply_update(Field out, Field in, Field r_prev, Field ap_prev, const double* alpha, const int* skip,
                              const int* gate, Field dot, int* nblocks)
     {
         (void)out; (void)in; (void)r_prev; (void)ap_prev; (void)alpha; (void)skip; (void)gate; (void)dot;
-        *nblocks = 0;
+        nblocks[0] = nblocks[1] = 0;
         return PPS_ERR_UNSUPPORTED;
     }
     // operator()(x, b) as the main solver on the context's X and B
@@ -585,12 +579,6 @@ struct KrylovStage : Stage {
         }
         return pre->apply_internal(out, in, gate);
     }
-    int pre_apply_dot(Field out, Field in, const int* gate, Field dot, int* nblocks)
-    {
-        *nblocks = 0;
-        if (!pre) return pre_apply(out, in, gate);
-        return pre->apply_dot(out, in, gate, dot, nblocks);
-    }
     // common prologue of the main/inner loop: returns 1 if the loop must not run
     int prologue(bool main, Field x, Field b, Field r, int* early)
     {
@@ -888,12 +876,12 @@ struct FCGStage : KrylovStage {
         auto body = [&]() -> int {
             if (fused_r) {
                 // iteration k: r_k = r_{k-1} - alpha_{k-1} Ap_{k-1} into rr[cur ^ 1]
-                int nb = 0;
+                int nb[2] = {0, 0};
                 int e = pre->apply_update(z, rr[cur ^ 1], rr[cur], Ap[cur ^ 1], &S->v[S_ALPHA], &S->restart, &S->done,
-                                          Ap[cur ^ 1], &nb);
+                                          Ap[cur ^ 1], nb);
                 if (e) return e;
-                if (nb > 0) launch_fcg_gamma_finish<double>(C.stream, C.rb, nb, S);
-                launch_fcg_gamma<double>(g, C.stream, C.rb, z.d(), Ap[cur ^ 1].d(), S, nb > 0);
+                if (nb[0] > 0) launch_fcg_gamma_finish<double>(C.stream, C.rb, nb[0], nb[1], S);
+                else launch_fcg_gamma<double>(g, C.stream, C.rb, z.d(), Ap[cur ^ 1].d(), S);
                 if (nring) {
                     const int qs = q % nring, qo = (q + nring - 1) % nring;
                     launch_fcg_p_fused<double>(g, C.stream, C.rb, z.d(), ring[qo].d(), ring[qs].d(), Ap[cur].d(),
@@ -907,12 +895,9 @@ struct FCGStage : KrylovStage {
                 cur ^= 1;
                 return PPS_OK;
             }
-            // the learned preconditioner sums z . Ap_old in its output kernel
-            int nb = 0;
-            int e = pre_apply_dot(z, r, &S->done, Ap[cur ^ 1], &nb);
+            int e = pre_apply(z, r, &S->done);
             if (e) return e;
-            if (nb > 0) launch_fcg_gamma_finish<double>(C.stream, C.rb, nb, S);
-            launch_fcg_gamma<double>(g, C.stream, C.rb, z.d(), Ap[cur ^ 1].d(), S, nb > 0);
+            launch_fcg_gamma<double>(g, C.stream, C.rb, z.d(), Ap[cur ^ 1].d(), S);
             launch_fcg_p<double>(g, C.stream, C.rb, z.d(), p[cur ^ 1].d(), p[cur].d(), Ap[cur].d(), r.d(), x.d(), S);
             launch_fcg_update<double>(g, C.stream, C.rb, r.d(), Ap[cur].d(), S, main);
             cur ^= 1;
@@ -974,12 +959,17 @@ __global__ void k_fallback(T* out, const T* in, Layout L, Region R, T c, const i
 }
 
 // the same with the residual update folded in: in = r_prev - alpha ap_prev
-// (r_prev while *skip) is formed, written and preconditioned
+// (r_prev while *skip) is formed, written and preconditioned, and out . ap_prev
+// summed into one partial per block (part != null): the Krylov step's gamma.  A
+// gated launch costs an iteration 2-4 us, so the fallback is this one kernel and
+// its sums take the same finish as the network's.
 template <typename T>
 __global__ void k_fallback_upd(T* out, T* in, const T* r_prev, const T* ap_prev, const double* alpha, const int* skip,
-                               Layout L, Region R, T c, const int* done, const int* fallback)
+                               Layout L, Region R, T c, const int* done, const int* fallback, double* part)
 {
     if (*done || !*fallback) return;
+    __shared__ double red[4];
+    double acc = 0.0;
     const T al = (T)*alpha;
     const bool sk = *skip != 0;
     const int n0 = R.hi[0] - R.lo[0], n1 = R.hi[1] - R.lo[1], n2 = R.hi[2] - R.lo[2];
@@ -988,10 +978,17 @@ __global__ void k_fallback_upd(T* out, T* in, const T* r_prev, const T* ap_prev,
         const int i = (int)(t % n0);
         const long long q = t / n0;
         const long long o = L.at(R.lo[0] + i, R.lo[1] + (int)(q % n1), R.lo[2] + (int)(q / n1));
-        const T r = sk ? r_prev[o] : r_prev[o] - al * ap_prev[o];
+        const T ap = ap_prev[o];
+        const T r = sk ? r_prev[o] : r_prev[o] - al * ap;
         in[o] = r;
         out[o] = c * r;
+        acc += (double)(c * r) * (double)ap;
     }
+    if (part == nullptr) return;
+    for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // a preconditioner is called with gate = &caller->done of the Krylov stage it
@@ -1019,12 +1016,8 @@ struct NNStage : Stage {
     long long iters_per_call() const override { return 1; }
     int apply(Field out, Field in, const int* gate) override
     {
-        int nb;
-        return apply_dot(out, in, gate, Field{}, &nb);
-    }
-    int apply_dot(Field out, Field in, const int* gate, Field dot, int* nblocks) override
-    {
-        return run(out, in, gate, dot, nullptr, nblocks);
+        int nb[2];
+        return run(out, in, gate, Field{}, nullptr, nb);
     }
     bool forms_update() const override { return true; }
     int apply_update(Field out, Field in, Field r_prev, Field ap_prev, const double* alpha, const int* skip,
@@ -1034,13 +1027,13 @@ struct NNStage : Stage {
         const NNResUpdate u{r_prev.p, ap_prev.p, in.p, alpha, skip};
         return run(out, in, gate, dot, &u, nblocks);
     }
-    // dot.p set: the output kernel also writes per-block partials of out . dot
-    // to the context's reduction workspace (gated like the network itself).
+    // dot.p set (ap_prev where u is): the output kernel, or the fallback, also writes
+    // per-block partials of out . dot to the context's reduction workspace.
     // u set: the network's lift (or the fallback) forms `in` from the residual
     // update first
     int run(Field out, Field in, const int* gate, Field dot, const NNResUpdate* u, int* nblocks)
     {
-        *nblocks = 0;
+        nblocks[0] = nblocks[1] = 0;
         if (!C.nn) return C.fail(PPS_ERR_STATE, "PPS_NN stage without a network (pps_nn_attach)");
         if (!gate) return C.fail(PPS_ERR_STATE, "PPS_NN stage called outside a Krylov stage");
         if (out.prec != in.prec) return C.fail(PPS_ERR_ARG, "PPS_NN: input and output precision differ");
@@ -1054,21 +1047,25 @@ struct NNStage : Stage {
         g.n0 = C.solver.hi[0] - C.solver.lo[0];
         g.n1 = C.solver.hi[1] - C.solver.lo[1];
         g.n2 = C.solver.hi[2] - C.solver.lo[2];
-        if (dot.p && dot.prec != out.prec) return C.fail(PPS_ERR_ARG, "PPS_NN: dot field precision differs");
+        if (dot.p && (dot.prec != out.prec || (u && dot.p != u->ap_prev))) return C.fail(PPS_ERR_ARG, "PPS_NN: bad dot field");
         if (C.nn->apply_dot(C.stream, g, out.p, out.prec, in.p, in.prec, &caller->done, &caller->fallback,
                             &caller->v[S_RR], dot.p, C.rb.partials, C.rb.cap, nblocks, u))
             return C.fail(PPS_ERR_HIP, "learned preconditioner: %s", C.nn->error());
         const double* ds = C.grid.ds;
         const double jac = 1.0 / (-2.0 * (1.0 / (ds[0] * ds[0]) + 1.0 / (ds[1] * ds[1]) + 1.0 / (ds[2] * ds[2])));
         if (u) {
+            const long long n = (long long)g.n0 * g.n1 * g.n2;
+            const int fb = (int)std::max<long long>(1, std::min<long long>({2048, C.rb.cap, (n + 255) / 256}));
+            double* part = nblocks[0] > 0 ? C.rb.partials : nullptr;
+            nblocks[1] = fb;
             if (in.prec == 32)
-                hipLaunchKernelGGL(k_fallback_upd<float>, dim3(2048), dim3(256), 0, C.stream, out.f(), in.f(),
+                hipLaunchKernelGGL(k_fallback_upd<float>, dim3(fb), dim3(256), 0, C.stream, out.f(), in.f(),
                                    (const float*)u->r_prev, (const float*)u->ap_prev, u->alpha, u->skip, L, C.solver,
-                                   (float)jac, &caller->done, &caller->fallback);
+                                   (float)jac, &caller->done, &caller->fallback, part);
             else
-                hipLaunchKernelGGL(k_fallback_upd<double>, dim3(2048), dim3(256), 0, C.stream, out.d(), in.d(),
+                hipLaunchKernelGGL(k_fallback_upd<double>, dim3(fb), dim3(256), 0, C.stream, out.d(), in.d(),
                                    (const double*)u->r_prev, (const double*)u->ap_prev, u->alpha, u->skip, L, C.solver,
-                                   jac, &caller->done, &caller->fallback);
+                                   jac, &caller->done, &caller->fallback, part);
         } else if (in.prec == 32) {
             hipLaunchKernelGGL(k_fallback<float>, dim3(2048), dim3(256), 0, C.stream, out.f(), in.f(), L, C.solver,
                                (float)jac, &caller->done, &caller->fallback);
@@ -1145,11 +1142,6 @@ struct IRStage : KrylovStage {
             return PPS_OK;
         };
         // the learned preconditioner sums z . Ap_old in its output kernel
-        auto applyM_dot = [&](const int* gate, Field dot, int* nb) -> int {
-            *nb = 0;
-            if (M) return M->apply_dot(z, r32, gate, dot, nb);
-            return applyM(gate);
-        };
         if (!flexible && !pw) {
             rc = applyM(&SI->done);
             if (rc) return rc;
@@ -1158,12 +1150,12 @@ struct IRStage : KrylovStage {
         rc = run_loop(C, SI, in->cfg.max_iter, host_each, [&]() -> int {
             if (fused_r) {
                 // iteration k: r_k = r_{k-1} - alpha_{k-1} Ap_{k-1} into rr[cur ^ 1]
-                int nb = 0;
+                int nb[2] = {0, 0};
                 int e = M->apply_update(z, rr[cur ^ 1], rr[cur], Ap[cur ^ 1], &SI->v[S_ALPHA], &SI->restart, &SI->done,
-                                        Ap[cur ^ 1], &nb);
+                                        Ap[cur ^ 1], nb);
                 if (e) return e;
-                if (nb > 0) launch_fcg_gamma_finish<float>(C.stream, C.rb, nb, SI);
-                launch_fcg_gamma<float>(g, C.stream, C.rb, z.f(), Ap[cur ^ 1].f(), SI, nb > 0);
+                if (nb[0] > 0) launch_fcg_gamma_finish<float>(C.stream, C.rb, nb[0], nb[1], SI);
+                else launch_fcg_gamma<float>(g, C.stream, C.rb, z.f(), Ap[cur ^ 1].f(), SI);
                 if (nring) {
                     const int qs = q % nring, qo = (q + nring - 1) % nring;
                     launch_fcg_p_fused<float>(g, C.stream, C.rb, z.f(), ring[qo].f(), ring[qs].f(), Ap[cur].f(),
@@ -1176,11 +1168,9 @@ struct IRStage : KrylovStage {
                 }
                 cur ^= 1;
             } else if (flexible) {
-                int nb = 0;
-                int e = applyM_dot(&SI->done, Ap[cur ^ 1], &nb);
+                int e = applyM(&SI->done);
                 if (e) return e;
-                if (nb > 0) launch_fcg_gamma_finish<float>(C.stream, C.rb, nb, SI);
-                launch_fcg_gamma<float>(g, C.stream, C.rb, z.f(), Ap[cur ^ 1].f(), SI, nb > 0);
+                launch_fcg_gamma<float>(g, C.stream, C.rb, z.f(), Ap[cur ^ 1].f(), SI);
                 launch_fcg_p<float>(g, C.stream, C.rb, z.f(), p[cur ^ 1].f(), p[cur].f(), Ap[cur].f(), r32.f(), d.f(), SI);
                 launch_fcg_update<float>(g, C.stream, C.rb, r32.f(), Ap[cur].f(), SI, false);
                 cur ^= 1;
@@ -2522,9 +2512,10 @@ int pps_nn_apply_field_prec(void* ctx, int out, int in, int prec, int dot, doubl
     pps_stage st{};
     st.kind = PPS_NN;
     NNStage stage(*C, st, 1);
-    int nblocks = 0;
-    rc = stage.apply_dot(ao, ai, &S->done, dot >= 0 ? ad : Field{}, &nblocks);
+    int nb2[2];
+    rc = stage.run(ao, ai, &S->done, dot >= 0 ? ad : Field{}, nullptr, nb2);
     if (rc) return rc;
+    const int nblocks = nb2[0];
     if (prec == 32) hipLaunchKernelGGL(k_widen, dim3(nb), dim3(256), 0, C->stream, ao.f(), fo.d(), n);
     if (dot < 0) return C->hip(hipStreamSynchronize(C->stream), "sync");
     if (nblocks <= 0) return C->fail(PPS_ERR_STATE, "pps_nn_apply_field_prec: the output layer formed no dot partials");
@@ -2577,8 +2568,8 @@ int pps_nn_apply_update(void* ctx, int out, int r_prev, int ap_prev, int r_cur, 
     pps_stage st{};
     st.kind = PPS_NN;
     NNStage stage(*C, st, 1);
-    int nblocks = 0;
-    rc = stage.apply_update(ao, ac, ap, aa, &S->v[S_ALPHA], &S->restart, &S->done, Field{}, &nblocks);
+    int nblocks[2];
+    rc = stage.apply_update(ao, ac, ap, aa, &S->v[S_ALPHA], &S->restart, &S->done, Field{}, nblocks);
     if (rc) return rc;
     if (prec == 32) {
         hipLaunchKernelGGL(k_widen, dim3(nb), dim3(256), 0, C->stream, ao.f(), fo.d(), n);

@@ -180,9 +180,8 @@ __device__ __forceinline__ void block_partials(double (&v)[NQ], const RedBuf& rb
 // interleaved accumulators (more loads in flight), then a fixed tree.
 constexpr int kFinThreads = 1024;
 template <int NQ, class Op>
-__global__ __launch_bounds__(kFinThreads) void k_finish(Op op, RedBuf rb, int nblocks)
+__device__ __forceinline__ void finish_block(Op& op, const RedBuf& rb, int nblocks)
 {
-    if (op.gated()) return;
     double a0[NQ], a1[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) a0[q] = a1[q] = 0.0;
@@ -203,6 +202,19 @@ __global__ __launch_bounds__(kFinThreads) void k_finish(Op op, RedBuf rb, int nb
     for (int q = 0; q < NQ; ++q) acc[q] = a0[q] + a1[q];
     block_sum<NQ, kFinThreads>(acc, tot);
     if (threadIdx.x == 0) op.finish(tot);
+}
+template <int NQ, class Op>
+__global__ __launch_bounds__(kFinThreads) void k_finish(Op op, RedBuf rb, int nblocks)
+{
+    if (op.gated()) return;
+    finish_block<NQ>(op, rb, nblocks);
+}
+// the same of nalt partials while *alt != 0
+template <int NQ, class Op>
+__global__ __launch_bounds__(kFinThreads) void k_finish_alt(Op op, RedBuf rb, int nblocks, int nalt, const int* alt)
+{
+    if (op.gated()) return;
+    finish_block<NQ>(op, rb, *alt ? nalt : nblocks);
 }
 
 struct Gate {
@@ -436,27 +448,6 @@ __global__ __launch_bounds__(VecShape<Op>::BT) void k_vector(Geo g, Op op, RedBu
                                              (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)));
 }
 
-// The same pass on a fixed grid of at most kStridedBlocks blocks, each taking
-// segments blockIdx.x, blockIdx.x + gridDim.x, ...: for passes that are
-// usually gated off (a gated one-shot launch still dispatches one block per
-// segment, ~0.1 ms at 512^3 for nothing), at some cost when they do run.
-constexpr int kStridedBlocks = 2048;
-template <int NQ, class Op, bool NT>
-__global__ __launch_bounds__(VecShape<Op>::BT) void k_vector_strided(Geo g, Op op, RedBuf rb, int nseg, int ny,
-                                                                     long long nb)
-{
-    if (op.gated()) return;
-    op.load();
-    double acc[NQ > 0 ? NQ : 1];
-#pragma unroll
-    for (int q = 0; q < (NQ > 0 ? NQ : 1); ++q) acc[q] = 0.0;
-    for (long long b = blockIdx.x; b < nb; b += gridDim.x) {
-        const long long rw = b / nseg;
-        vector_segment<NT>(g, op, (int)(b - rw * nseg), g.lo1 + (int)(rw % ny), g.lo2 + (int)(rw / ny), acc);
-    }
-    if constexpr (NQ > 0) block_partials<NQ, VecShape<Op>::BT>(acc, rb, (int)blockIdx.x);
-}
-
 // sums of kSpan consecutive block partials, one block per span, fixed order
 template <int NQ, class Op>
 __global__ __launch_bounds__(kThreads) void k_span(Op op, RedBuf rb, int nblocks)
@@ -533,7 +524,7 @@ static void run_stencil(const Geo& g0, hipStream_t s, const Op& op, RedBuf rb)
 }
 
 template <int NQ, class Op>
-static void run_vector(const Geo& g0, hipStream_t s, const Op& op, RedBuf rb, bool strided = false)
+static void run_vector(const Geo& g0, hipStream_t s, const Op& op, RedBuf rb)
 {
     const int nx = g0.hi0 - g0.lo0, ny = g0.hi1 - g0.lo1, nz = g0.hi2 - g0.lo2;
     if (nx <= 0 || ny <= 0 || nz <= 0) return;
@@ -545,15 +536,6 @@ static void run_vector(const Geo& g0, hipStream_t s, const Op& op, RedBuf rb, bo
         return;
     }
     Geo g = g0;
-    if (strided) {
-        g.nblocks = (int)std::min<long long>(nb, kStridedBlocks);
-        if (!check_capacity<NQ, Op>(g, rb)) return;
-        const dim3 grid(g.nblocks), block(VecShape<Op>::BT);
-        if (g.nt) hipLaunchKernelGGL((k_vector_strided<NQ, Op, true>), grid, block, 0, s, g, op, rb, nseg, ny, nb);
-        else hipLaunchKernelGGL((k_vector_strided<NQ, Op, false>), grid, block, 0, s, g, op, rb, nseg, ny, nb);
-        if constexpr (NQ > 0) launch_finish<NQ>(s, op, rb, g.nblocks);
-        return;
-    }
     g.nblocks = (int)nb;
     if (!check_capacity<NQ, Op>(g, rb)) return;
     const dim3 grid(nseg, ny, nz);
@@ -2262,21 +2244,17 @@ __device__ inline void update_finish(Scal* S, double rr, bool history)
     }
 }
 
-// gamma = z.Apold and beta.  When the preconditioner sums z.Apold itself (the
-// learned one, from its output kernel), only the finish runs, gated off once
-// the fallback preconditioner has taken over; the pass over z and Apold then
-// runs only while the fallback is on.
+// gamma = z.Apold and beta.  Where the preconditioner sums z.Apold itself (the
+// learned one in its output kernel, its fallback in its update), only the finish
+// runs.  With a pass over z and Apold and a second finish for the fallback, gated
+// off in nearly every iteration, an iteration had two launches more (learned FCG
+// solves, us: FP64 66^3 2999 / 2906 without them, 130^3 4770 / 4701; under
+// refinement 34^3 3862 / 3655).
 template <typename T>
 struct OpFcgGamma : Gate {
     const T* __restrict__ z;
     const T* __restrict__ Apold;
     Scal* S;
-    const int* skip_if = nullptr;  // gated while *skip_if != 0
-    const int* run_if = nullptr;   // gated while *run_if == 0
-    __device__ __forceinline__ bool gated() const
-    {
-        return Gate::gated() || (skip_if && *skip_if) || (run_if && !*run_if);
-    }
     struct R { T z, a; };
     __device__ void load() {}
     template <bool NT> __device__ R fetch(long long c) const { return {ld<NT>(z + c), ld<NT>(Apold + c)}; }
@@ -2290,28 +2268,27 @@ struct OpFcgGamma : Gate {
 };
 
 template <typename T>
-void launch_fcg_gamma(const Geo& g, hipStream_t s, RedBuf rb, const T* z, const T* Apold, Scal* S, bool fallback_only)
+void launch_fcg_gamma(const Geo& g, hipStream_t s, RedBuf rb, const T* z, const T* Apold, Scal* S)
 {
     OpFcgGamma<T> op;
     op.gate = &S->done;
     op.z = z;
     op.Apold = Apold;
     op.S = S;
-    if (fallback_only) op.run_if = &S->fallback;
-    run_vector<1>(g, s, op, rb, fallback_only);
+    run_vector<1>(g, s, op, rb);
 }
 
 template <typename T>
-void launch_fcg_gamma_finish(hipStream_t s, RedBuf rb, int nblocks, Scal* S)
+void launch_fcg_gamma_finish(hipStream_t s, RedBuf rb, int nblocks, int nfallback, Scal* S)
 {
     OpFcgGamma<T> op;
     op.gate = &S->done;
     op.z = nullptr;
     op.Apold = nullptr;
     op.S = S;
-    op.skip_if = &S->fallback;
     if (nblocks <= 0 || nblocks > rb.cap) return;
-    hipLaunchKernelGGL((k_finish<1, OpFcgGamma<T>>), dim3(1), dim3(kFinThreads), 0, s, op, rb, nblocks);
+    hipLaunchKernelGGL((k_finish_alt<1, OpFcgGamma<T>>), dim3(1), dim3(kFinThreads), 0, s, op, rb, nblocks, nfallback,
+                       &S->fallback);
 }
 
 // p = z - beta pold ; Ap = A p ; p.Ap, p.r ; alpha = p.r / p.Ap ; and the
@@ -2706,8 +2683,8 @@ void launch_ir_inner_init(const Geo& g, hipStream_t s, RedBuf rb, float* r, floa
                                      const T*, const T*, Scal*, bool);                                         \
     template void launch_bicg_k6<T>(const Geo&, hipStream_t, T*, const T*, const T*, const Scal*);             \
     template void launch_cheb_first<T>(const Geo&, hipStream_t, const T*, T*, T*, double, double, const int*); \
-    template void launch_fcg_gamma<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, Scal*, bool);       \
-    template void launch_fcg_gamma_finish<T>(hipStream_t, RedBuf, int, Scal*);                                  \
+    template void launch_fcg_gamma<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, Scal*);             \
+    template void launch_fcg_gamma_finish<T>(hipStream_t, RedBuf, int, int, Scal*);                             \
     template void launch_fcg_p<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, T*, T*, const T*, T*, Scal*); \
     template void launch_fcg_p_fused<T>(const Geo&, hipStream_t, RedBuf, const T*, const T*, T*, T*, const T*, T*,    \
                                         Scal*, bool, int);                                                         \
