@@ -1366,15 +1366,36 @@ __global__ __launch_bounds__(256) void k_repitch(double* __restrict__ dense, dou
     }
 }
 
+// clears the pending error that a tolerated failure has just left, but not one
+// that was there before it (an earlier launch's, not reported yet)
+static void drop_error(hipError_t before)
+{
+    if (before == hipSuccess) (void)hipGetLastError();
+}
+
 // whether `host` is ordinary pageable memory (not allocated or registered through HIP)
 static bool pageable(const void* host)
 {
+    const hipError_t before = hipPeekAtLastError();
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, host) != hipSuccess) {
-        (void)hipGetLastError();
+        drop_error(before);
         return true;
     }
     return at.type == hipMemoryTypeUnregistered;
+}
+
+// k_repitch of nk planes from plane k0; the launch's own status, since neither the
+// copies around it nor a stream synchronisation report a launch that was refused
+template <bool UP>
+static hipError_t repitch(Ctx& C, double* field, int k0, int nk)
+{
+    double* dense = C.stage_d;
+    Layout L = C.L64;
+    long long rows = (long long)nk * C.ng[1];
+    void* args[] = {&dense, &field, &L, &k0, &rows};
+    return hipLaunchKernel(reinterpret_cast<const void*>(&k_repitch<UP>),
+                           dim3((unsigned)std::min<long long>((rows + 3) / 4, 8192)), dim3(256), args, 0, C.stream);
 }
 
 // host array <-> field.  Pinned memory takes one pitched copy (57 GB/s, the
@@ -1392,10 +1413,11 @@ static int transfer(Ctx& C, int field, double* host, bool up)
     const bool staged = pageable(host);
     if (staged && !C.stage_d) {
         const int np = (int)std::min<size_t>(C.ng[2], std::max<size_t>(1, kStageBytes / (plane * sizeof(double))));
+        const hipError_t before = hipPeekAtLastError();
         if (hipMalloc(&C.stage_d, np * plane * sizeof(double)) == hipSuccess) {
             C.stage_planes = np;
         } else {
-            (void)hipGetLastError();  // no room: the row-by-row copy below still works
+            drop_error(before);  // no room: the row-by-row copy below still works
             C.stage_d = nullptr;
         }
     }
@@ -1403,14 +1425,12 @@ static int transfer(Ctx& C, int field, double* host, bool up)
         for (int k0 = 0; k0 < C.ng[2]; k0 += C.stage_planes) {
             const int nk = std::min(C.stage_planes, C.ng[2] - k0);
             const size_t bytes = nk * plane * sizeof(double);
-            const long long rows = (long long)nk * C.ng[1];
-            const dim3 grid((unsigned)std::min<long long>((rows + 3) / 4, 8192));
             double* h = host + k0 * plane;
             if (up) {
                 if ((rc = C.hip(hipMemcpyAsync(C.stage_d, h, bytes, hipMemcpyHostToDevice, C.stream), "upload"))) return rc;
-                hipLaunchKernelGGL(k_repitch<true>, grid, dim3(256), 0, C.stream, C.stage_d, f.d(), C.L64, k0, rows);
+                if ((rc = C.hip(repitch<true>(C, f.d(), k0, nk), "upload repitch"))) return rc;
             } else {
-                hipLaunchKernelGGL(k_repitch<false>, grid, dim3(256), 0, C.stream, C.stage_d, f.d(), C.L64, k0, rows);
+                if ((rc = C.hip(repitch<false>(C, f.d(), k0, nk), "download repitch"))) return rc;
                 if ((rc = C.hip(hipMemcpyAsync(h, C.stage_d, bytes, hipMemcpyDeviceToHost, C.stream), "download"))) return rc;
             }
         }
