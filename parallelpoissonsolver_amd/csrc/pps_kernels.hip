@@ -2077,7 +2077,12 @@ __global__ __launch_bounds__(kTX* kChW, RY == 2 && !(NEU && S == 3) ? 4 : 2) voi
                 return lap7(P.uc, u[row][col - 1], u[row][col + 1], u[row - 1][col], u[row + 1][col], P.um, P.un, cx, cy, cz);
             };
             T Av[RY];
-            if (!NEU || !ghosts) {
+            // the pass's last level is wanted on the solver region only: ghost positions
+            // take no mirror there (a mirrored centre may lie a column or row before the
+            // tile, whose neighbours level 1 of a two-sweep pass does not hold)
+            constexpr bool kMir2 = NEU && S == 3;
+            static_assert(!kMir2 || S - 1 >= 2, "a mirrored centre's neighbours lie in level 1's planes");
+            if (!kMir2 || !ghosts) {
 #pragma unroll
                 for (int q = 0; q < RY; ++q) {
                     const int row = jr + q + S - 1, col = lx + S - 1;
