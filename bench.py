@@ -177,15 +177,17 @@ def host_cpu():
 def cpu_baseline(gpu_iterations):
     """Reference CPU solver (compiled from the reference sources into oracle/_ref)
     on the host cores: 100 CG iterations of the same 512^3 workload under MPI,
-    extrapolated to the iteration count the solve needs.  None, with a line in the
-    log, where the reference build or mpirun is missing (pass --no-cpu to skip the
-    baseline)."""
+    extrapolated to the iteration count the solve needs.  Where the reference build
+    or mpirun is missing there is no value but the reason ("skipped"), which a run
+    without the baseline (--no-cpu: null) does not have."""
     exe = os.path.join(ROOT, "oracle", "_ref", "ref_solver_sample")
     mpirun = shutil.which("mpirun") or "/opt/conda/bin/mpirun"
     if not (os.path.exists(exe) and os.path.exists(mpirun)):
-        log(f"CPU baseline: not measured, {exe} or mpirun missing (build with __graft_entry__.build() where the "
-            f"reference sources are present)")
-        return None
+        missing = [what for what, path in (("the reference build oracle/_ref/ref_solver_sample", exe),
+                                           ("mpirun", mpirun)) if not os.path.exists(path)]
+        log(f"CPU baseline: not measured, missing: {', '.join(missing)} (__graft_entry__.build() builds the reference "
+            f"where its sources are present)")
+        return {"value": None, "unit": "s", "skipped": "missing: " + ", ".join(missing)}
     npg = N_INTERIOR + 2
     ds = 1.0 / (npg - 1)
     ranks = (2, 2, 2)  # 514 = 2 * 257: the reference needs ranks dividing npglobal (blockGrid.hpp:165)
