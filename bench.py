@@ -111,7 +111,7 @@ def run_form(C, chain, steps, warmup, name):
 
 KERNELS = {"cg_stencil_f64": 0, "cg_update_f64": 1, "residual_f64": 2, "copy_f64": 3, "cheb_sweep_f64": 4,
            "cg_stencil_f32": 5, "cg_update_f32": 6, "fcg_stencil_f64": 7, "fcg_stencil_f32": 8,
-           "copy_flat_f64": 9, "cheb_pair_f64": 10}  # PPS_K_* ids of include/pps_abi.h
+           "copy_flat_f64": 9, "cheb_pair_f64": 10, "cg_pass_f64": 11, "cg_pass_f32": 12, "cheb_triple_f64": 13}  # PPS_K_* ids of include/pps_abi.h
 
 
 def profiled_traffic(kernel, n):
@@ -288,16 +288,17 @@ def main():
     # dominant kernel of the headline solve: largest device time per iteration.
     # Per learned-FCG iteration: one network apply (each layer once; the output
     # layer also sums gamma and the lift forms the residual update) and the
-    # fused FCG p-stencil pass; per plain-CG iteration: the fused stencil and
-    # update.
+    # fused FCG p-stencil pass; per plain-CG iteration: the one pass of it.
     if headline in ("ir_nnfcg", "nn_fcg_fp64"):
         per_it = {f"nn_{k}": v for k, v in layers.items()}
         sfx = "f32" if headline == "ir_nnfcg" else "f64"
         per_it[f"fcg_stencil_{sfx}"] = kern[f"fcg_stencil_{sfx}"]
     elif headline == "ir_fp32cg_fp64":
-        per_it = {k: kern[k] for k in ("cg_stencil_f32", "cg_update_f32")}
+        per_it = {"cg_pass_f32": kern["cg_pass_f32"]}
+    elif headline == "plain_fp64_cg":
+        per_it = {"cg_pass_f64": kern["cg_pass_f64"]}
     else:
-        per_it = {k: kern[k] for k in ("cg_stencil_f64", "cg_update_f64")}
+        per_it = {"cheb_triple_f64": kern["cheb_triple_f64"]}
     dom = max(per_it, key=lambda k: per_it[k]["ms"])
     k = per_it[dom]
     roof = {"bound": "hbm", "kernel": dom, "achieved": round(k["gbs"], 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
@@ -343,13 +344,16 @@ def main():
         "nn_layers": {k2: {"gbs": round(v["gbs"], 1), "tflops": round(v["tflops"], 2), "ms": round(v["ms"], 4)}
                       for k2, v in layers.items()},
         "roofline": roof,
-        # Chebyshev sweeps at this size: one per launch (4 fields) and two fused per launch (5 fields)
+        # Chebyshev sweeps at this size: one per launch (4 fields), two or three fused per launch (5 fields); the
+        # solver runs them three per pass, its first one or two passes with two
         "chebyshev": ({"single_sweep_ms": round(kern["cheb_sweep_f64"]["ms"], 4),
                        "single_sweep_gbs": round(kern["cheb_sweep_f64"]["gbs"], 1),
                        "pair_ms": round(kern["cheb_pair_f64"]["ms"], 4),
                        "pair_gbs": round(kern["cheb_pair_f64"]["gbs"], 1),
-                       "per_sweep_ms_fused": round(kern["cheb_pair_f64"]["ms"] / 2, 4)}
-                      if "cheb_pair_f64" in kern else None),
+                       "triple_ms": round(kern["cheb_triple_f64"]["ms"], 4),
+                       "triple_gbs": round(kern["cheb_triple_f64"]["gbs"], 1),
+                       "per_sweep_ms_fused": round(kern["cheb_triple_f64"]["ms"] / 3, 4)}
+                      if "cheb_triple_f64" in kern else None),
         "cpu_baseline": cpu,
     }
     print(json.dumps(out), flush=True)

@@ -206,7 +206,11 @@ enum {
     PPS_K_FCG_STENCIL_F32 = 8,
     PPS_K_COPY_FLAT = 9,       /* plain 1-D copy of a whole field allocation (16-byte
                                   non-temporal lanes): the measured HBM ceiling */
-    PPS_K_CHEB_PAIR = 10       /* two fused Chebyshev sweeps: read Y, Z, B ; write y_{c+1}, y_{c+2} */
+    PPS_K_CHEB_PAIR = 10,      /* two fused Chebyshev sweeps: read Y, Z, B ; write y_{c+1}, y_{c+2} */
+    PPS_K_CG_PASS = 11,        /* CG with a pointwise preconditioner: one iteration, read r, p ; write
+                                  r, p (x's updates deferred as above) */
+    PPS_K_CG_PASS_F32 = 12,
+    PPS_K_CHEB_TRIPLE = 13     /* three fused Chebyshev sweeps: read Y, Z, B ; write the last two */
 };
 /* Average device time (ms) of `reps` back-to-back launches of one kernel on
  * the context stream, measured with HIP events; *bytes = algorithmic bytes

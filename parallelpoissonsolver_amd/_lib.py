@@ -18,7 +18,7 @@ ERRORS = {-1: "PPS_ERR_ARG", -2: "PPS_ERR_HIP", -3: "PPS_ERR_NOMEM", -4: "PPS_ER
 FIELD_X, FIELD_B, FIELD_T0, FIELD_T1, FIELD_T2, FIELD_T3 = range(6)
 NONE, CG, BICGSTAB, CHEBYSHEV, JACOBI, FCG, IR, NN = range(8)
 (K_CG_STENCIL, K_CG_UPDATE, K_RESIDUAL, K_COPY, K_CHEB_SWEEP, K_CG_STENCIL_F32, K_CG_UPDATE_F32, K_FCG_STENCIL,
- K_FCG_STENCIL_F32, K_COPY_FLAT, K_CHEB_PAIR) = range(11)
+ K_FCG_STENCIL_F32, K_COPY_FLAT, K_CHEB_PAIR, K_CG_PASS, K_CG_PASS_F32, K_CHEB_TRIPLE) = range(14)
 
 
 class PPSError(RuntimeError):

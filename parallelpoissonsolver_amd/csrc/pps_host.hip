@@ -2046,7 +2046,8 @@ int pps_time_kernel(void* ctx, int kernel, int reps, double* ms, double* bytes)
 {
     Ctx* C = as_ctx(ctx);
     if (!C || reps < 1 || !ms || !bytes) return PPS_ERR_ARG;
-    const int P = (kernel == PPS_K_CG_STENCIL_F32 || kernel == PPS_K_CG_UPDATE_F32 || kernel == PPS_K_FCG_STENCIL_F32)
+    const int P = (kernel == PPS_K_CG_STENCIL_F32 || kernel == PPS_K_CG_UPDATE_F32 || kernel == PPS_K_FCG_STENCIL_F32 ||
+                   kernel == PPS_K_CG_PASS_F32)
                       ? 32 : 64;
     const double w = P == 32 ? 4.0 : 8.0;
     const double n = (double)C->solver.count();
@@ -2100,13 +2101,21 @@ int pps_time_kernel(void* ctx, int kernel, int reps, double* ms, double* bytes)
                                       d.f(), f.f(), e.f(), S, false, 0);
             break;
         case PPS_K_COPY_FLAT: launch_copy_flat(C->stream, a.d(), e.d(), C->L64.total); break;
-        case PPS_K_CHEB_PAIR: {
-            const double ca[2] = {0.1, 0.15}, cb[2] = {0.2, 0.25}, cc[2] = {0.3, 0.35};
-            launch_cheb_multi<double, double>(g, C->cheb_pair_geo(), C->stream, 2, (it & 1) ? d.d() : a.d(), b.d(), c.d(),
-                                              (it & 1) ? e.d() : d.d(), (it & 1) ? a.d() : e.d(), ca, cb, cc, 1.0, 1.0,
-                                              1.0, nullptr);
+        case PPS_K_CHEB_PAIR: case PPS_K_CHEB_TRIPLE: {
+            const double ca[3] = {0.1, 0.15, 0.12}, cb[3] = {0.2, 0.25, 0.22}, cc[3] = {0.3, 0.35, 0.32};
+            launch_cheb_multi<double, double>(g, C->cheb_pair_geo(), C->stream, kernel == PPS_K_CHEB_PAIR ? 2 : 3,
+                                              (it & 1) ? d.d() : a.d(), b.d(), c.d(), (it & 1) ? e.d() : d.d(),
+                                              (it & 1) ? a.d() : e.d(), ca, cb, cc, 1.0, 1.0, 1.0, nullptr);
             break;
         }
+        case PPS_K_CG_PASS:
+            launch_cg_pass<double>(g, C->stream, C->rb, (it & 1) ? b.d() : a.d(), (it & 1) ? f.d() : c.d(),
+                                   (it & 1) ? a.d() : b.d(), (it & 1) ? c.d() : f.d(), e.d(), S, false, 0);
+            break;
+        case PPS_K_CG_PASS_F32:
+            launch_cg_pass<float>(g, C->stream, C->rb, (it & 1) ? b.f() : a.f(), (it & 1) ? f.f() : c.f(),
+                                  (it & 1) ? a.f() : b.f(), (it & 1) ? c.f() : f.f(), e.f(), S, false, 0);
+            break;
         }
     };
     double per = 0;
@@ -2118,7 +2127,8 @@ int pps_time_kernel(void* ctx, int kernel, int reps, double* ms, double* bytes)
     case PPS_K_CHEB_SWEEP: per = 4; break;                              // read Y, B, Z ; write W
     case PPS_K_FCG_STENCIL: case PPS_K_FCG_STENCIL_F32: per = 5; break; // read z, p_old, r ; write p, Ap
     case PPS_K_COPY_FLAT: per = 2.0 * (double)C->L64.total / n; break;  // the whole allocation, read and written
-    case PPS_K_CHEB_PAIR: per = 5; break;                               // read Y, Z, B ; write W1, W2 (two sweeps)
+    case PPS_K_CHEB_PAIR: case PPS_K_CHEB_TRIPLE: per = 5; break;       // read Y, Z, B ; write the last two levels
+    case PPS_K_CG_PASS: case PPS_K_CG_PASS_F32: per = 4; break;         // read r, p ; write r, p
     default: return C->fail(PPS_ERR_ARG, "unknown kernel id %d", kernel);
     }
     for (int i = 0; i < 3; ++i) launch(i);  // warm-up

@@ -1,7 +1,43 @@
 """bench.py's record, as far as it can be checked without a GPU."""
 import os
+import re
+
+import pytest
 
 import bench
+from tests.conftest import ROOT
+
+
+def header_kernels():
+    text = open(os.path.join(ROOT, "include", "pps_abi.h")).read()
+    return {name: int(v) for name, v in re.findall(r"\bPPS_K_(\w+) = (\d+)", text)}
+
+
+def test_kernel_ids_are_the_headers():
+    from parallelpoissonsolver_amd import _lib
+    ids = header_kernels()
+    assert sorted(bench.KERNELS.values()) == sorted(ids.values()) == list(range(len(ids)))
+    for name, v in ids.items():
+        assert getattr(_lib, "K_" + name) == v
+
+
+def test_the_timed_kernels_are_the_ones_that_run():
+    """Plain CG's pass and the three-sweep Chebyshev pass are among the timed kernels."""
+    ids = header_kernels()
+    for name, key in (("cg_pass_f64", "CG_PASS"), ("cg_pass_f32", "CG_PASS_F32"), ("cheb_triple_f64", "CHEB_TRIPLE")):
+        assert bench.KERNELS[name] == ids[key]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,bytes_per_point", [("cg_pass_f64", 32), ("cg_pass_f32", 16), ("cheb_triple_f64", 40)])
+def test_timing_of_the_passes(name, bytes_per_point):
+    import parallelpoissonsolver_amd._lib as L
+    C = L.Context((67, 50, 35), (0.1, 0.1, 0.1))
+    ms, nbytes = C.time_kernel(bench.KERNELS[name], 3)
+    assert ms > 0 and nbytes == bytes_per_point * 65 * 48 * 33
+    with pytest.raises(L.PPSError):
+        C.time_kernel(len(bench.KERNELS), 1)
+    C.close()
 
 
 def test_a_missing_cpu_baseline_says_why(tmp_path, monkeypatch):
