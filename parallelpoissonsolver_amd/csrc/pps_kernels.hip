@@ -1033,7 +1033,17 @@ __device__ __forceinline__ void ring_point(int t, int& r, int& c)
     else { r = t - 2 * (W + 2) - H; c = W; }
 }
 
-constexpr int kCUs = 256;  // compute units of the MI355X
+int cu_count()
+{
+    static const int n = [] {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+            return v;
+        return 256;
+    }();
+    return n;
+}
 
 // z-chunk of a marching kernel whose blocks take kz + extra steps and of which
 // per_cu (1 or 2) fit on a CU: the one with the least time on the busiest CU (the
@@ -1044,9 +1054,10 @@ static int pick_kz(long long tiles, int nz, int per_cu, int extra)
 {
     int best = 1;
     double cost = -1.0;
+    const int cus = cu_count();
     for (int kz = 1; kz <= 128; ++kz) {
         if (kz > 1 && kz > nz) break;
-        const long long n = (tiles * ((nz + kz - 1) / kz) + kCUs - 1) / kCUs;  // blocks of the busiest CU
+        const long long n = (tiles * ((nz + kz - 1) / kz) + cus - 1) / cus;  // blocks of the busiest CU
         const double c = (per_cu == 2 ? (n / 2) * 1.5 + n % 2 : (double)n) * (std::min(kz, nz) + extra);
         if (cost < 0.0 || c <= cost) {
             cost = c;
@@ -1340,7 +1351,7 @@ void launch_cg_pass(const Geo& g0, hipStream_t s, RedBuf rb, const T* r_in, cons
     // blocks per CU) below that.  us per iteration, 32 / 16 rows, FP64: 514^3
     // 1110 / 1169, 258^3 145 / 148, 194^3 77.5 / 71.5, 130^3 32.8 / 27.1, 66^3 15.5 / 13.9
     // (and where the last row of 32-row tiles is more than half full)
-    const bool tall = tiles(4 * kCgW) * nz >= 2ll * 16 * kCUs && (ny - 1) % (4 * kCgW) + 1 > 2 * kCgW;
+    const bool tall = tiles(4 * kCgW) * nz >= 2ll * 16 * cu_count() && (ny - 1) % (4 * kCgW) + 1 > 2 * kCgW;
     if (tall) run_cg_pass<T, 4>(tiling(4 * kCgW, 1), s, A, op, rb);
     else run_cg_pass<T, 2>(tiling(2 * kCgW, 2), s, A, op, rb);
 }
@@ -2225,7 +2236,7 @@ void launch_cheb_multi(const Geo& g, const ChebPairGeo& cg, hipStream_t s, int s
     // 131x257x190 (256 rows) 1796 / 1859, 258^3 (257 rows) 4334 / 3997
     const int nx = g.hi0 - g.lo0, ny = g.hi1 - g.lo1, nz = g.hi2 - g.lo2, tail = (ny - 1) % (4 * kChW) + 1;
     const long long tiles = (long long)((nx + kTX - 1) / kTX) * ((ny + 4 * kChW - 1) / (4 * kChW));
-    const bool tall = tiles * nz >= 8ll * kCUs && tail > 2 * kChW;
+    const bool tall = tiles * nz >= 8ll * cu_count() && tail > 2 * kChW;
     if (sweeps == 3 && tall) run_cheb_multi<T, TO, 3, 4>(g, cg, s, A, 1);
     else if (sweeps == 3) run_cheb_multi<T, TO, 3, 2>(g, cg, s, A, cg.neu && sizeof(T) == 8 ? 1 : 2);
     else if (tall) run_cheb_multi<T, TO, 2, 4>(g, cg, s, A, 1);

@@ -108,6 +108,8 @@ struct Geo {
 
 // kz_st: z-chunk length of the stencil kernels; nt: non-temporal stores
 Geo make_geo(const Layout& L, const Region& R, const double coef[3], int kz_st, int nt);
+// compute units of the device (256 on an MI355X in one partition; also where it cannot be asked)
+int cu_count();
 
 // Neumann faces of the current grid, for the ghost-fill kernel.
 struct Faces {

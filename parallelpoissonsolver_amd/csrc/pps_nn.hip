@@ -14,6 +14,7 @@
 // LDS and marches along z with a ring of 4 planes, one barrier per plane.
 // Each of the 4 wavefronts computes 4 x-rows of 16 voxels per plane.
 #include "pps_nn.hpp"
+#include "pps_kernels.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -1119,19 +1120,6 @@ static int pick_zc(int D, int H, int W, int B)
     while (zc > 16 && tiles * ((D + zc - 1) / zc) < 8192) zc = (zc + 1) / 2;
     if ((zc & 1) && zc < D) ++zc;  // chunks start on even planes (z pairs of the pooled lift output)
     return std::max(zc, 1);
-}
-static int cu_count()
-{
-    static int n = 0;
-    if (n == 0) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            n = v;
-        else
-            n = 256;
-    }
-    return n;
 }
 // z-chunk of the forward kernels that march z: the even one (or all of D) with
 // the least work for the busiest CU, blocks per CU times the chunk and its three
