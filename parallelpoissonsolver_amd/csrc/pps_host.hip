@@ -1141,7 +1141,6 @@ struct IRStage : KrylovStage {
             launch_pointwise<float>(C.gbox(32), C.stream, r32.f(), z.f(), 1.0, gate);
             return PPS_OK;
         };
-        // the learned preconditioner sums z . Ap_old in its output kernel
         if (!flexible && !pw) {
             rc = applyM(&SI->done);
             if (rc) return rc;
@@ -1562,11 +1561,13 @@ int pps_create(const pps_grid* grid, void** out)
     rc = rc ? rc : X.hip(hipEventCreate(&X.ev_t0), "event");
     rc = rc ? rc : X.hip(hipEventCreate(&X.ev_t1), "event");
     // reduction workspace: partials for the largest launch (a vector kernel
-    // over the whole box, or a stencil at the smallest z-chunk allowed), and
-    // the span sums of the two-level epilogue
+    // over the whole box, or a marching kernel at its smallest z-chunk; below, a
+    // stencil's at the smallest one a caller may set), and the span sums of the
+    // two-level epilogue
     const Geo gbig = make_geo(X.L64, X.box, X.coef, kMinKz, 0);
     const long long nvec = (long long)((X.ng[0] + kThreads - 1) / kThreads) * X.ng[1] * X.ng[2];
-    // one-plane chunks of 64 x 16 tiles (small grids' CG pass)
+    // one-plane chunks of 64 x 16 tiles: small grids' CG pass, and more than the
+    // two-plane chunks of 64 x 32 tiles of their stencils
     const long long nsmall = (long long)((X.ng[0] + kTX - 1) / kTX) * ((X.ng[1] + 15) / 16) * X.ng[2];
     // the network's output kernel: 14 x 16 tiles in chunks of 2 planes at least
     const long long nout = (long long)((X.ng[0] + 13) / 14) * ((X.ng[1] + 15) / 16) * ((X.ng[2] + 1) / 2);

@@ -4,7 +4,7 @@
 //  * k_stencil: 2.5-D z-marching tile.  A block of 64x8 threads owns a 64x32
 //    column tile (kTX x kTH: each thread four rows) of one x-y slab and marches
 //    through kz planes (the longest of 64/32/16/8 that still gives 2048
-//    blocks).  Each thread keeps its columns' (k-1, k, k+1) values in
+//    blocks; 4 or 2 on grids too small for 1024 blocks of 8).  Each thread keeps its columns' (k-1, k, k+1) values in
 //    registers; the plane-k tile and its one-point halo are staged in LDS
 //    (double-buffered, one barrier per plane), so x- and y-neighbours come from
 //    LDS and every value of the input field is produced once per plane (this is
@@ -1087,7 +1087,8 @@ static int pick_kz(long long tiles, int nz, int per_cu, int extra)
 // Measured at 512^3 FP64: 0.85 ms for its 4 words (5.06 TB/s; 5.4 with the rings'
 // re-reads that miss L2, 1.14x on the reads), where the stencil and update
 // passes took 0.83 + 0.53 ms; 1.10 against 1.60 ms per iteration with x's
-// deferred updates.  The HBM rate is that of the other marching stencils.
+// deferred updates.  The HBM rate is that of the other marching stencils.  FP32:
+// 0.47 ms (4.6 TB/s; 5.7 with the re-reads, 1.52x on the reads).
 //
 // A block owns a 64 x (8 RY) tile and marches z.  It forms p on the tile and a
 // one-point ring, from p_old on the tile and a two-point ring; a thread owns RY
@@ -1830,8 +1831,9 @@ void launch_cheb_sweep(const Geo& g, hipStream_t s, const T* Y, const T* B, cons
 // register.  A level's other points off the solver region are 0; B's, which the
 // first pass's start reads, are whatever the field holds there.
 //
-// Measured at 512^3 FP64: three sweeps in 1.27 ms (4.2 TB/s of its 5 words; 4.6
-// with the rings' re-reads that miss L2), 0.42 ms per sweep, where the pair took
+// Measured at 512^3 FP64: three sweeps in 1.24 ms (4.3 TB/s of its 5 words; 4.7
+// with the rings' re-reads that miss L2, 1.16x on the reads; vector pipe 22 % busy,
+// LDS 16 %), 0.41 ms per sweep, where the pair took
 // 1.08 ms and needed a ghost fill per pass with Neumann faces.  On grids that stay
 // in the caches the steps' instructions are half of the time, so plane pointers
 // are advanced instead of formed from the plane's number and two steps make a trip

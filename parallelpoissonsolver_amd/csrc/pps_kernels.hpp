@@ -32,7 +32,7 @@ constexpr int kSTY = PPS_STENCIL_WAVES;
 constexpr int kSThreads = kTX * kSTY;
 constexpr int kTH = kSTY * kRY;  // stencil tile height (rows)
 constexpr int kMaxRedQ = 5;
-constexpr int kMinKz = 4;   // smallest z-chunk; sizes the reduction workspace
+constexpr int kMinKz = 4;   // smallest z-chunk that a caller may set (the kernels' own rules go down to one plane)
 
 struct Layout {
     int ng[3];        // guarded extent per direction
@@ -174,8 +174,13 @@ void launch_ghost(hipStream_t s, const Layout& L, const Faces& F, T* field, int 
 // ---- CG with a pointwise preconditioner: one pass per iteration ----
 // One launch is one iteration (see k_cg_pass): r_out = r_in - alpha_prev A pin,
 // pout = jac r_out + beta pin, A pout and the iteration's sums, whose finish
-// sets alpha, beta, the residual norm and the convergence flag.  r_in/r_out
-// and pin/pout must be distinct buffers holding 0 off the solver region.
+// sets alpha, beta, the residual norm and the convergence flag.  That norm, and
+// with it beta, the history and the iteration's reported error, is predicted:
+// sqrt(r.r - 2 alpha r.Ap + alpha^2 Ap.Ap) of this pass's sums stands for the sum
+// over the next residual, to a relative error of about eps / kCgRecheck in ||r||^2
+// at most (2e-14 in FP64; below kCgRecheck r.r the sum itself is taken).  r_in/r_out
+// and pin/pout must be distinct buffers; nothing is read or written off the solver
+// region, where every value counts as 0.
 // ring_slot >= 0: alpha goes to S->ahist[ring_slot] for launch_fcg_flush and x
 // is not touched; otherwise x += alpha_prev pin (the caller adds the last step).
 // The buffers alternate with S->passes: pass n (from 0) reads what pass n - 1 wrote.
@@ -238,10 +243,10 @@ struct ChebPairGeo {
 // `sweeps` = 2 or 3 fused sweeps: W = the last one's y (sign-applied and
 // converted to TO), Wp = the one before (null: not written).  Y = y_c and
 // Z = y_{c-1}; Z = null: the recurrence's start, Y = B, whose first level is
-// c1 (2B + c0 AB) (a[0], b[0], c[0] unused; B's values off the solver region
-// take part, its Neumann ghosts must be set).  Otherwise nothing is read off the
-// solver region: the levels' Neumann ghosts are formed in the kernel, their
-// other points there count as 0.  40 rows of a field must be smaller than 2 GiB.
+// c1 (2B + c0 AB) (a[0], b[0], c[0] unused).  Neumann ghosts, B's and every
+// level's, are formed in the kernel from their mirror points and never read; B's
+// other values off the solver region take part in the start, every level's count
+// as 0 there.  40 rows of a field must be smaller than 2 GiB.
 template <typename T, typename TO>
 void launch_cheb_multi(const Geo& g, const ChebPairGeo& cg, hipStream_t s, int sweeps, const T* Y, const T* Z, const T* B,
                        T* Wp, TO* W, const double* a, const double* b, const double* c, double c0, double c1, double sign,

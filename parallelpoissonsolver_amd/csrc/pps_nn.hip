@@ -1127,7 +1127,10 @@ static int pick_zc(int D, int H, int W, int B)
 // them faster, so fewer count as `fill`.  `keep` (or 0) is a chunk that was tuned
 // on large grids, kept unless the model promises 15 % (at 384^3 the model's choice
 // for level 1 is 3 % slower).  No result depends on the chunk (the output kernel's
-// partials of z . dot aside).  us per launch, chunks of 16 planes (the least there
+// partials of z . dot aside).  Where the chunks already give a CU two blocks the
+// model moves little: level 2 of 512^3 (8 picked, 16 kept before) 32.2 / 32.7 us in
+// the layers' timing loop and 29.8 / 29.4 in the solve, of 320^3 (2; 10) 11.8 / 12.8.
+// us per launch, chunks of 16 planes (the least there
 // was) / as picked: level 2 of 256^3 16.5 / 7.8 (2 planes); level 1 of 128^3 16.6 /
 // 8.0 (2); lift at 128^3 20.4 / 12.4 (4); output kernel at 64^3 20.6 / 11.7 (2), at
 // 256^3 155 / 145 (32)
@@ -1261,9 +1264,10 @@ void launch_lift(const ConvArgs& a, hipStream_t s)
 // differ from it by that rounding (relative ~1e-3 at most) and FP32 order.
 // Rows outside the domain are masked in the tiles that have any; the other tiles
 // run a copy of the march without masks.
-// Bound: issue and latency, not memory (2.1 GB a pass at 512^3).  A plane of a
-// wavefront is 24 MFMAs (384 cycles), about 75 vector instructions (300) and 14
-// LDS reads in about 820 cycles.  The form before it summed nine row partials per
+// Bound: issue, not memory (2.1 GB a pass at 512^3).  A plane of a wavefront is 24
+// MFMAs (384 cycles), about 75 vector instructions (300) and 14 LDS reads.  Counters:
+// matrix pipe 57 % busy, vector pipe 49 %, both at once 23 %, so one or the other 83 %
+// of the time; LDS 70 %, without bank conflicts.  The form before it summed nine row partials per
 // voxel through LDS (9 reads, 40 DPP moves and 113 vector instructions per plane):
 // us per call with the gamma operand, 512^3 FP32 978 -> 880, 256^3 FP64 (gated
 // calls counted) 92 -> 84.  Occupancy decides: 3 blocks per CU 955 us; 5 blocks
